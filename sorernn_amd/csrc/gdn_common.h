@@ -77,6 +77,11 @@ __device__ __forceinline__ float silu_fast(float x) {
   return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
 }
 
+// The logistic function by the same two instructions (for gradients rounded to a 16-bit type).
+__device__ __forceinline__ float sigmoid_fast(float x) {
+  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
+}
+
 // ---------------------------------------------------------------- wave reductions
 __device__ __forceinline__ float wave_xor_sum(float x, int from_stride) {
   for (int s = from_stride; s < kWave; s <<= 1) x += __shfl_xor(x, s, kWave);
@@ -91,16 +96,21 @@ __device__ __forceinline__ float dpp_add(float v) {
   return v + __int_as_float(s);
 }
 
-// Sum over aligned groups of N lanes (N = 8 or 16) with DPP: quad_perm [1,0,3,2] and [2,3,0,1]
+// Sum over aligned groups of N lanes (N = 8, 16 or 32) with DPP: quad_perm [1,0,3,2] and [2,3,0,1]
 // (0xb1, 0x4e), row_half_mirror (0x141, pairs the two quads of an 8-lane half) and row_mirror
-// (0x140, pairs the two halves of a 16-lane row). Every lane of a group ends with the group sum.
+// (0x140, pairs the two halves of a 16-lane row), then gfx950's 16-lane swap of row pairs. Every
+// lane of a group ends with the group sum.
 template <int N>
 __device__ __forceinline__ float group_sum(float x) {
-  static_assert(N == 8 || N == 16, "group of 8 or 16 lanes");
+  static_assert(N == 8 || N == 16 || N == 32, "group of 8, 16 or 32 lanes");
   x = dpp_add<0xb1, 0xf>(x);
   x = dpp_add<0x4e, 0xf>(x);
   x = dpp_add<0x141, 0xf>(x);
-  if (N == 16) x = dpp_add<0x140, 0xf>(x);
+  if (N >= 16) x = dpp_add<0x140, 0xf>(x);
+  if (N == 32) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
   return x;
 }
 

@@ -1,0 +1,58 @@
+"""GPU: the vector backward of the L2 norm and of the (gated) RMSNorm at the edges of its tiles.
+
+Against fp64 autograd on the same inputs. The bound per element is one rounding of the result to its
+type (half a unit in the last place) plus 2^-20 of the row's largest term for the fp32 arithmetic; the
+fp32 parameter gradients, sums over all rows, are bounded by 2^-20 of the sum of their terms' magnitudes.
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from sorernn_amd import l2norm, rms_norm_gated
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# relative to the value: 8, 11 and 24 significant bits (a value just above 2^k has units of 2^(k-7), 2^(k-10), 2^(k-23))
+HALF_ULP = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 2.0**-24}
+
+
+def _check(name, got, ref, row_scale):
+    err = (got.double().cpu() - ref).abs()
+    # subnormal fp16 results round to a fixed step of 2^-24
+    bound = HALF_ULP[got.dtype] * ref.abs() * 1.01 + 2.0**-20 * row_scale + (2.0**-25 if got.dtype == torch.float16 else 0)
+    assert (err <= bound).all(), f"{name}: {(err / bound).max().item():.2f} of the bound"
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("rows", [1, 3, 17, 64, 1025, 70001])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_norm_backwards_at_tile_edges(dtype, rows, d):
+    gen = torch.Generator().manual_seed(rows + d)
+    x, g, dy = (torch.randn(rows, d, generator=gen).to(dtype) for _ in range(3))
+    w, b = torch.randn(d, generator=gen), 0.1 * torch.randn(d, generator=gen)
+    xr = x.double().requires_grad_(True)
+    xd = x.to(DEV).requires_grad_(True)
+    (ref,) = torch.autograd.grad(F.normalize(xr, dim=-1), xr, dy.double())
+    (got,) = torch.autograd.grad(l2norm(xd), xd, dy.to(DEV))
+    _check("l2 dx", got, ref, (dy.double().abs().amax(-1, keepdim=True) / x.double().norm(dim=-1, keepdim=True)))
+    for act, bias, gated in (("swish", None, True), (None, b, True), ("swish", b, False)):
+        lv = [x, g, w] + ([b] if bias is not None else [])
+        rf = [t.double().requires_grad_(True) for t in lv]
+        rr = torch.rsqrt(rf[0].square().mean(-1, keepdim=True) + 1e-6)
+        u = rf[0] * rr * rf[2] + (rf[3] if bias is not None else 0)
+        y = u * (F.silu(rf[1]) if act else rf[1]) if gated else u
+        dev = [t.to(DEV).requires_grad_(True) for t in lv]
+        yd = rms_norm_gated(dev[0], dev[1] if gated else None, dev[2], dev[3] if bias is not None else None, activation=act)
+        pick = [0] + ([1] if gated else []) + [2] + ([3] if bias is not None else [])
+        refs = torch.autograd.grad(y, [rf[i] for i in pick], dy.double())
+        gots = torch.autograd.grad(yd, [dev[i] for i in pick], dy.to(DEV))
+        gate = (F.silu(rf[1]) if act else rf[1]).detach() if gated else torch.ones(1, dtype=torch.double)
+        du = dy.double() * gate
+        top = lambda t: t.abs().amax(-1, keepdim=True)  # noqa: E731
+        n, rd = (rf[0] * rr).detach(), rr.detach()
+        scale = {0: rd * top(du * rf[2].detach()) * (1 + top(n)) ** 2, 2: (du * n).abs().sum(0), 3: du.abs().sum(0)}
+        # u = n w + b can cancel: its fp32 error is relative to the two terms, not to their sum
+        u_terms = (n * rf[2].detach()).abs() + (b.double().abs() if bias is not None else 0)
+        scale[1] = dy.double().abs() * u_terms * (1 + g.double().abs())
+        for i, a, r in zip(pick, gots, refs):
+            _check(f"rms {act} gated={gated} grad {i}", a, r, scale[i])
