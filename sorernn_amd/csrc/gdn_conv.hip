@@ -349,7 +349,7 @@ struct ConvBwdParams {
   int64_t T, C, N;
   int dx_t, act;
   void* dx;
-  float* part;   // [blocks][C][W + 1]
+  float* part;   // [blocks][W + 1][C]
   float* dinit;  // [N][C][W] fp32, zeroed first, or null
 };
 
@@ -440,22 +440,206 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_bwd_kernel(ConvBwdPara
     if (pos >= t0 && pos < t1) store_from_f32(p.dx, p.dx_t, (row + pos) * p.C + c, pend[i]);
   }
   const int64_t blk = bb * gridDim.y + blockIdx.y;
-  float* pp = p.part + (blk * p.C + c) * (W + 1);
+  float* pp = p.part + blk * (W + 1) * p.C + c;
 #pragma unroll
-  for (int i = 0; i < W; ++i) pp[i] = dw[i];
-  pp[W] = db;
+  for (int i = 0; i < W; ++i) pp[i * p.C] = dw[i];
+  pp[W * p.C] = db;
 }
 
-// dweight [C][W] and dbias [C] (fp32) from the per-block partial sums [blocks][C][W + 1].
-__global__ __launch_bounds__(256) void gated_delta_conv1d_param_grad_kernel(const float* part, int64_t blocks, int64_t C,
-                                                                            int W, float* dw, float* dbias) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;  // = c * (W + 1) + i
-  if (e >= C * (W + 1)) return;
+// Vector path of the backward for W = 4 and C % 4 == 0: a thread owns 4 consecutive channels (8-byte
+// accesses of 16-bit types, 16-byte of fp32) and walks `tt` tokens plus the 3 after them, the x and dy rows
+// of 4 tokens loaded before the first is used. HBM-bound: x and dy in, dx out. The four waves of a workgroup
+// take consecutive token segments of the same 256 channels, so the segments' overlapping rows meet in the
+// cache and one row of dw/dbias partial sums leaves per workgroup (added over the waves in LDS) instead of
+// one per segment. 4 channels and not 8, so that the per-channel state (weights, window, pending dx, dw: 17
+// values) leaves room for 4 waves per SIMD. 16,384 tokens x 2,048 channels in bf16, 24 documents: 49 us (4.1 TB/s) against 146
+// with one channel per thread (the kernel above, kept for other W, C and alignments).
+template <typename E>
+__global__ __launch_bounds__(256) void gated_delta_conv1d_bwd_vec_kernel(ConvBwdParams p, int tt) {
+  constexpr int W = 4, V = 4, G = 4;
+  typedef E VE __attribute__((ext_vector_type(V)));
+  constexpr bool kFast = sizeof(E) == 2;  // results rounded to 16 bits: sigmoid from v_exp_f32 / v_rcp_f32
+  __shared__ __align__(16) float red[4][W + 1][kWave * V];
+  const int lane = threadIdx.x % kWave, wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const unsigned c0 = (blockIdx.x * kWave + lane) * V;
+  const int64_t bb = blockIdx.z;
+  const int T = (int)p.T, t0 = ((int)blockIdx.y * 4 + wv) * tt;
+  const int t1 = t0 + tt < T ? t0 + tt : T, tend = t1 + W - 1 < T ? t1 + W - 1 : T;
+  float dw[W][V], db[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    db[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < W; ++i) dw[i][e] = 0.f;
+  }
+  if (c0 < p.C && t0 < T) {
+    // row bases are the same for the whole wave (scalar registers), the lane's channel is a 32-bit offset
+    const E* __restrict__ xs = static_cast<const E*>(p.x) + bb * p.T * p.C;
+    const E* __restrict__ dys = static_cast<const E*>(p.dy) + bb * p.T * p.C;
+    E* __restrict__ dxs = static_cast<E*>(p.dx) + bb * p.T * p.C;
+    const E* init = static_cast<const E*>(p.init);
+    float w[V][W], bias[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+#pragma unroll
+      for (int i = 0; i < W; ++i) w[e][i] = p.w[(c0 + e) * W + i];
+      bias[e] = p.bias ? p.bias[c0 + e] : 0.f;
+    }
+    int d = (int)bb, ds = 0, de = T;  // the document that holds token t: [ds, de), the same for the whole wave
+    if (p.cu) {
+      int lo = 0, hi = (int)p.N - 1;  // largest d with cu[d] <= t0
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (__builtin_amdgcn_readfirstlane((int)load_index(p.cu, p.cu_i32, mid)) <= t0) lo = mid;
+        else hi = mid - 1;
+      }
+      d = lo;
+      ds = __builtin_amdgcn_readfirstlane((int)load_index(p.cu, p.cu_i32, d));
+      de = __builtin_amdgcn_readfirstlane((int)load_index(p.cu, p.cu_i32, d + 1));
+    }
+    float win[W - 1][V];  // inputs at t - 3 + i
+#pragma unroll
+    for (int i = 0; i < W - 1; ++i) {
+      const int pos = t0 - (W - 1) + i;
+      if (pos >= ds) {
+        const VE v = *reinterpret_cast<const VE*>(xs + (int64_t)pos * p.C + c0);
+#pragma unroll
+        for (int e = 0; e < V; ++e) win[i][e] = (float)v[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+          win[i][e] = init ? (float)init[((int64_t)d * p.C + c0 + e) * W + (W - (ds - pos))] : 0.f;
+      }
+    }
+    float pend[W - 1][V];  // dx of the positions t - 3 + i so far
+#pragma unroll
+    for (int i = 0; i < W - 1; ++i)
+#pragma unroll
+      for (int e = 0; e < V; ++e) pend[i][e] = 0.f;
+    auto store_dx = [&](int pos, const float (&v)[V]) {
+      VE o;
+#pragma unroll
+      for (int e = 0; e < V; ++e) o[e] = (E)v[e];
+      *reinterpret_cast<VE*>(dxs + (int64_t)pos * p.C + c0) = o;
+    };
+    for (int tg = t0; tg < tend; tg += G) {
+      VE xv[G], dv[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {  // rows past tend re-read the last one (never used)
+        const int64_t at = (int64_t)(tg + g < tend ? tg + g : tend - 1) * p.C;
+        xv[g] = *reinterpret_cast<const VE*>(xs + at + c0);
+        dv[g] = *reinterpret_cast<const VE*>(dys + at + c0);
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const int t = tg + g;
+        if (t >= tend) break;
+        while (t >= de) {  // next document: restart the window from its initial state
+          ++d;
+          ds = de;
+          de = __builtin_amdgcn_readfirstlane((int)load_index(p.cu, p.cu_i32, d + 1));
+#pragma unroll
+          for (int i = 0; i < W - 1; ++i)
+#pragma unroll
+            for (int e = 0; e < V; ++e) win[i][e] = init ? (float)init[((int64_t)d * p.C + c0 + e) * W + i + 1] : 0.f;
+        }
+        float xt[V], dz[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          xt[e] = (float)xv[g][e];
+          float z = bias[e] + w[e][W - 1] * xt[e];
+#pragma unroll
+          for (int i = 0; i < W - 1; ++i) z += w[e][i] * win[i][e];
+          dz[e] = (float)dv[g][e];
+          if (p.act == GDN_ACT_SILU) {
+            const float sg = kFast ? sigmoid_fast(z) : sigmoid_f32(z);
+            dz[e] *= sg * (1.f + z * (1.f - sg));
+          }
+        }
+        if (t < t1) {  // the halo's tokens belong to the next segment's dw
+#pragma unroll
+          for (int e = 0; e < V; ++e) {
+            dw[W - 1][e] += dz[e] * xt[e];
+            db[e] += dz[e];
+#pragma unroll
+            for (int i = 0; i < W - 1; ++i) dw[i][e] += dz[e] * win[i][e];
+          }
+        }
+        if (t - ds >= W - 1) {
+#pragma unroll
+          for (int i = 0; i < W - 1; ++i)
+#pragma unroll
+            for (int e = 0; e < V; ++e) pend[i][e] += w[e][i] * dz[e];
+        } else {  // positions before the document take nothing from it (never multiplied by 0: dz may be NaN)
+#pragma unroll
+          for (int i = 0; i < W - 1; ++i) {
+            const int pos = t - (W - 1) + i;
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+              if (pos >= ds) pend[i][e] += w[e][i] * dz[e];
+              else if (p.dinit && t < t1) atomicAdd(&p.dinit[((int64_t)d * p.C + c0 + e) * W + (W - (ds - pos))], w[e][i] * dz[e]);
+            }
+          }
+        }
+        if (t - (W - 1) >= t0) store_dx(t - (W - 1), pend[0]);
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          pend[0][e] = pend[1][e];
+          pend[1][e] = pend[2][e];
+          pend[2][e] = w[e][W - 1] * dz[e];
+          win[0][e] = win[1][e];
+          win[1][e] = win[2][e];
+          win[2][e] = xt[e];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < W - 1; ++i) {  // the last positions of the sequence, which nothing follows
+      const int pos = tend - (W - 1) + i;
+      if (pos >= t0 && pos < t1) store_dx(pos, pend[i]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+#pragma unroll
+    for (int i = 0; i < W; ++i) red[wv][i][lane * V + e] = dw[i][e];
+    red[wv][W][lane * V + e] = db[e];
+  }
+  __syncthreads();
+  float* pp = p.part + (bb * gridDim.y + blockIdx.y) * (W + 1) * p.C + (int64_t)blockIdx.x * kWave * V;
+  const int64_t left = p.C - (int64_t)blockIdx.x * kWave * V;
+  for (int k = 0; k <= W; ++k) {
+    const int c = threadIdx.x;  // kWave * V = 256 columns, one per thread
+    if (c < left) pp[k * p.C + c] = (red[0][k][c] + red[1][k][c]) + (red[2][k][c] + red[3][k][c]);
+  }
+}
+
+// dweight [C][W] and dbias [C] (fp32) from the partial sums [blocks][W + 1][C]: one workgroup per 64
+// columns, 16 rows of partial sums at a time, then the 16 row lanes in LDS (4 us for 128 rows of
+// 5 x 2,048 columns; one thread per column, the rows in order, took 60 us for 256).
+constexpr int kConvParamCols = 64, kConvParamLanes = 16;
+
+__global__ __launch_bounds__(kConvParamCols* kConvParamLanes) void gated_delta_conv1d_param_grad_kernel(
+    const float* __restrict__ part, int64_t blocks, int64_t C, int W, float* dw, float* dbias) {
+  __shared__ float red[kConvParamLanes][kConvParamCols];
+  const int ci = threadIdx.x % kConvParamCols, rl = threadIdx.x / kConvParamCols;
+  const int64_t cols = C * (W + 1), e = (int64_t)blockIdx.x * kConvParamCols + ci;  // = i * C + c
   float acc = 0.f;
-  for (int64_t b = 0; b < blocks; ++b) acc += part[b * C * (W + 1) + e];
-  const int64_t c = e / (W + 1), i = e % (W + 1);
-  if (i < W) dw[c * W + i] = acc;
-  else if (dbias) dbias[c] = acc;
+  if (e < cols) {
+#pragma unroll 8
+    for (int64_t b = rl; b < blocks; b += kConvParamLanes) acc += part[b * cols + e];
+  }
+  red[rl][ci] = acc;
+  __syncthreads();
+  for (int s = kConvParamLanes / 2; s > 0; s >>= 1) {
+    if (rl < s) red[rl][ci] += red[rl + s][ci];
+    __syncthreads();
+  }
+  if (rl == 0 && e < cols) {
+    const int64_t i = e / C, c = e % C;
+    if (i < W) dw[c * W + i] = red[0][ci];
+    else if (dbias) dbias[c] = red[0][ci];
+  }
 }
 
 __global__ void gated_delta_fill_zero_kernel(float* p, int64_t n) {
@@ -569,22 +753,42 @@ extern "C" int gdn_causal_conv1d_bwd(const void* x, const float* weight, const f
   }
   ConvBwdParams p{x, weight, bias, dy, initial_state, cu_seqlens, (flags & GDN_FLAG_CU_INT32) ? 1 : 0, T, C, N,
                   x_dtype, activation, dx, static_cast<float*>(workspace), initial_state ? d_initial_state : nullptr};
-  dim3 grid((unsigned)((C + 255) / 256), (unsigned)tb, (unsigned)B), block(256);
-  switch (W) {
-    case 1: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<1>, grid, block, 0, s, p); break;
-    case 2: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<2>, grid, block, 0, s, p); break;
-    case 3: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<3>, grid, block, 0, s, p); break;
-    case 4: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<4>, grid, block, 0, s, p); break;
-    case 5: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<5>, grid, block, 0, s, p); break;
-    case 6: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<6>, grid, block, 0, s, p); break;
-    case 7: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<7>, grid, block, 0, s, p); break;
-    default: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<8>, grid, block, 0, s, p); break;
+  const size_t esz = x_dtype == GDN_DTYPE_F32 ? 4 : 2;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) |
+                         reinterpret_cast<uintptr_t>(dx)) & (4 * esz - 1)) == 0;
+  int64_t parts = B * tb;  // rows of partial sums
+  if (aligned && W == 4 && C % 4 == 0) {
+    // Tokens per wave: the longest segment (fewest overlapping rows and partial sums) that still gives 4,096
+    // waves, the 4 per SIMD that the kernel's registers allow. Both launches, bf16, us at 16 / 32 / 64 / 128
+    // tokens: 16,384 x 4,096 102 / 94.5 / 92.8 / 100.6; 16,384 x 2,048 49.5 / 45.9 / 53.8 / 81.5; 4,096 x 2,048
+    // 19.5 / 23.8 / 37.5 / 67.3. Not below 16: 4 x 16 tokens a workgroup is the 64-token block that the
+    // workspace counts, and 8 tokens measured 19.1 at the last shape.
+    int tt = 64;
+    while (tt > 16 && B * ((T + tt - 1) / tt) * ((C + 255) / 256) < 4096) tt /= 2;
+    const dim3 gv((unsigned)((C + 255) / 256), (unsigned)((T + 4 * tt - 1) / (4 * tt)), (unsigned)B);
+    parts = (int64_t)gv.y * B;
+    if (x_dtype == GDN_DTYPE_BF16) hipLaunchKernelGGL(gated_delta_conv1d_bwd_vec_kernel<bf16>, gv, dim3(256), 0, s, p, tt);
+    else if (x_dtype == GDN_DTYPE_F16) hipLaunchKernelGGL(gated_delta_conv1d_bwd_vec_kernel<f16>, gv, dim3(256), 0, s, p, tt);
+    else hipLaunchKernelGGL(gated_delta_conv1d_bwd_vec_kernel<float>, gv, dim3(256), 0, s, p, tt);
+  } else {
+    dim3 grid((unsigned)((C + 255) / 256), (unsigned)tb, (unsigned)B), block(256);
+    switch (W) {
+      case 1: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<1>, grid, block, 0, s, p); break;
+      case 2: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<2>, grid, block, 0, s, p); break;
+      case 3: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<3>, grid, block, 0, s, p); break;
+      case 4: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<4>, grid, block, 0, s, p); break;
+      case 5: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<5>, grid, block, 0, s, p); break;
+      case 6: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<6>, grid, block, 0, s, p); break;
+      case 7: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<7>, grid, block, 0, s, p); break;
+      default: hipLaunchKernelGGL(gated_delta_conv1d_bwd_kernel<8>, grid, block, 0, s, p); break;
+    }
   }
   int rc = gdn_internal_check_launch("gated_delta_conv1d_bwd_kernel");
   if (rc != GDN_OK) return rc;
   const int64_t ne = C * (W + 1);
-  hipLaunchKernelGGL(gated_delta_conv1d_param_grad_kernel, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s,
-                     static_cast<const float*>(workspace), B * tb, C, (int)W, dweight, dbias);
+  hipLaunchKernelGGL(gated_delta_conv1d_param_grad_kernel, dim3((unsigned)((ne + kConvParamCols - 1) / kConvParamCols)),
+                     dim3(kConvParamCols * kConvParamLanes), 0, s, static_cast<const float*>(workspace), parts, C, (int)W,
+                     dweight, dbias);
   return gdn_internal_check_launch("gated_delta_conv1d_param_grad_kernel");
 }
 
