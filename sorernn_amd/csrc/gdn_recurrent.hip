@@ -1,15 +1,14 @@
-// Recurrent gated delta rule (token by token, state on chip) and the fused decode step.
+// Recurrent gated delta rule (state on chip in fp32, any number of tokens) and the fused decode step.
 //
-// One workgroup of 256 threads owns one (sequence, value head) state S [K, V] fp32 for the whole
-// sequence: it is read from HBM once, kept in registers (16 float4 per thread at K = V = 128) and
-// written once. Thread t owns the 4 columns 4*(t % (V/4)) .. +3 and the rows rg + RG*i, where
-// rg = t / (V/4) and RG = 256 / (V/4); the columns' dot products with k and q reduce over row groups
-// with a cross-lane xor reduction inside each wave and one LDS exchange across the 4 waves.
 // Per token (sore/model/gdn_ref.py:17-21):
-//   a = exp(g), S_dec = a S, delta = beta (v - S_dec^T k), S' = S_dec + k delta^T,
-//   o = scale S'^T q = scale (a S^T q + delta (k . q)),
-// so one pass over S yields S^T k and S^T q together (the state is read once per token).
-// No MFMA: per token the work is two matrix-vector products and a rank-1 update, bandwidth-bound.
+//   a = exp(g), S_dec = a S, delta = beta (v - S_dec^T k), S' = S_dec + k delta^T, o = scale S'^T q.
+// The state [K, V] fp32 of a (sequence, value head) is read from HBM once, kept in registers and written once.
+// Three kernels: gated_delta_recurrent_kernel takes 16 tokens at a time on fp32 MFMAs,
+// gated_delta_recurrent_short_kernel a few tokens one by one, gated_delta_decode_w4_kernel one token together
+// with the conv cache's step (gated_delta_decode_kernel for other conv widths and types, with the state in 256
+// threads: thread t owns the columns 4*(t % (V/4)) .. +3 and the rows rg + RG*i, rg = t / (V/4)).
+
+#include <type_traits>
 
 #include "gdn_common.h"
 #include "gdn_mfma.h"
@@ -131,13 +130,30 @@ __device__ __forceinline__ void store_state(const StateRegs<KD, VD>& sr, float* 
   for (int i = 0; i < L::RPT; ++i) *reinterpret_cast<float4*>(base + (int64_t)(rg + L::RG * i) * VD + 4 * cg) = s[i];
 }
 
-// grid (HV, N): one workgroup per (value head, sequence), tokens in order.
-template <int KD, int VD>
-__global__ __launch_bounds__(256) void gated_delta_recurrent_kernel(RecParams p) {
-  using L = RecLayout<KD, VD>;
-  __shared__ float stage[2][2 * KD + VD];
-  __shared__ float red[2][L::NW * L::CG * 12];
-  const int hv = blockIdx.x;
+template <typename E, int N>
+struct RowVec {
+  typedef E T __attribute__((ext_vector_type(N), aligned(sizeof(E))));  // rows may start at any element
+};
+
+constexpr int kShortTokens = 4;
+
+// The recurrence of a few tokens (a decode call, a draft of two or three): one pass over at most G = 4 tokens at a
+// time, all their loads issued at once. Columns of the state are independent (column j needs only S[:, j]), so
+// a wave owns 16 columns and nothing crosses waves: no LDS, no barrier. Lane (c4, rg) holds rows rg R ..
+// rg R + R - 1 (R = K / 16) of columns 4 c4 .. 4 c4 + 3; sums over rows stay inside a 16-lane DPP row. Gates and
+// q/k norms are computed with one token per lane and broadcast by readlane; lane rg stores token rg's outputs.
+// The state's bytes bound it from 16 sequences of 16 heads up: 64 sequences, T = 1, bf16, d = 128: 25.1 us (134 MB
+// of state, 5.3 TB/s); the kernel before it (one workgroup per state, two barriers a token) took 25.5, and 42.4
+// at T = 4 against 28.7 here.
+template <typename E, int KD, int VD>
+__global__ __launch_bounds__(256) void gated_delta_recurrent_short_kernel(RecParams p) {
+  constexpr int G = kShortTokens, R = KD / 16, NC = 4;
+  using VK = typename RowVec<E, R>::T;
+  using VV = typename RowVec<E, NC>::T;
+  using VS = typename RowVec<float, NC>::T;
+  const int lane = threadIdx.x % kWave, rg = lane % 16;
+  constexpr int kSlices = VD / 64;
+  const int hv = blockIdx.x / kSlices, col = (blockIdx.x % kSlices) * 64 + (threadIdx.x / 16) * NC;
   const int64_t n = blockIdx.y;
   const int h = hv / (int)(p.HV / p.H);
   int64_t bos, eos;
@@ -148,33 +164,356 @@ __global__ __launch_bounds__(256) void gated_delta_recurrent_kernel(RecParams p)
     bos = n * p.T;
     eos = bos + p.T;
   }
-  const int64_t sbase = (n * p.HV + hv) * (int64_t)KD * VD;
-  StateRegs<KD, VD> s;
-  load_state<KD, VD>(s, p.h0 ? p.h0 + sbase : nullptr);
-  const bool l2 = p.flags & GDN_FLAG_QK_L2NORM;
-  const int t = threadIdx.x;
-  int par = 0;
-  for (int64_t tok = bos; tok < eos; ++tok, par ^= 1) {
-    float* st = stage[par];
-    for (int e = t; e < 2 * KD + VD; e += L::NT) {
-      float x;
-      if (e < KD) x = load_as_f32(p.q, p.dq, (tok * p.H + h) * KD + e);
-      else if (e < 2 * KD) x = load_as_f32(p.k, p.dq, (tok * p.H + h) * KD + (e - KD));
-      else x = load_as_f32(p.v, p.dq, (tok * p.HV + hv) * VD + (e - 2 * KD));
-      st[e] = x;
-    }
-    float a, b;
-    gate_values(p, tok * p.HV + hv, hv, a, b);
-    __syncthreads();
-    float o4[4];
-    rec_token<KD, VD>(s, st, st + KD, st + 2 * KD, a, b, l2, p.scale, red[par], o4);
-    if (t < L::CG) {
-      const int64_t ob = (tok * p.HV + hv) * VD + 4 * t;
+  const int64_t sbase = (n * p.HV + hv) * (int64_t)KD * VD + (int64_t)rg * R * VD + col;
+  VS s[R];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) store_from_f32(p.o, p.dq, ob + c, o4[c]);
+  for (int i = 0; i < R; ++i) s[i] = p.h0 ? *reinterpret_cast<const VS*>(p.h0 + sbase + i * VD) : VS{};
+  const E* __restrict__ kp = static_cast<const E*>(p.k) + (int64_t)h * KD + rg * R;
+  const E* __restrict__ qp = static_cast<const E*>(p.q) + (int64_t)h * KD + rg * R;
+  const E* __restrict__ vp = static_cast<const E*>(p.v) + (int64_t)hv * VD + col;
+  E* __restrict__ op = static_cast<E*>(p.o) + (int64_t)hv * VD + col;
+  auto bcast = [](float x, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); };
+  for (int64_t t = bos; t < eos; t += G) {
+    VK k[G], q[G];
+    VV v[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {  // tokens past the end re-read the last one (never used)
+      const int64_t tok = t + g < eos ? t + g : eos - 1;
+      k[g] = *reinterpret_cast<const VK*>(kp + tok * p.H * KD);
+      q[g] = *reinterpret_cast<const VK*>(qp + tok * p.H * KD);
+      v[g] = *reinterpret_cast<const VV*>(vp + tok * p.HV * VD);
+    }
+    const int64_t gt = t + rg % G < eos ? t + rg % G : eos - 1;  // one token's gates per lane
+    float av, bv;
+    gate_values(p, gt * p.HV + hv, hv, av, bv);
+    float ikv = 1.f, iqv = p.scale;  // lane g: 1 / max(|k|, 1e-12) and scale / max(|q|, 1e-12) of token g
+    if (p.flags & GDN_FLAG_QK_L2NORM) {
+      float kkv = 0.f, qqv = 0.f;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        if (t + g >= eos) break;
+        float kk = 0.f, qq = 0.f;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          kk += (float)k[g][i] * (float)k[g][i];
+          qq += (float)q[g][i] * (float)q[g][i];
+        }
+        kk = group_sum<16>(kk);
+        qq = group_sum<16>(qq);
+        kkv = rg == g ? kk : kkv;
+        qqv = rg == g ? qq : qqv;
+      }
+      ikv = 1.f / fmaxf(sqrtf(kkv), 1e-12f);
+      iqv = p.scale / fmaxf(sqrtf(qqv), 1e-12f);
+    }
+    VV keep{};
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (t + g >= eos) break;
+      const float a = bcast(av, g), b = bcast(bv, g), ik = bcast(ikv, g), iq = bcast(iqv, g);
+      float kr[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) kr[i] = (float)k[g][i] * ik;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        float x = 0.f, o = 0.f;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          s[i][c] *= a;
+          x += s[i][c] * kr[i];
+        }
+        const float d = b * ((float)v[g][c] - group_sum<16>(x));
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          s[i][c] += kr[i] * d;
+          o += s[i][c] * (float)q[g][i];
+        }
+        o = group_sum<16>(o) * iq;
+        keep[c] = rg == g ? (E)o : keep[c];
+      }
+    }
+    if (rg < G && t + rg < eos) *reinterpret_cast<VV*>(op + (t + rg) * p.HV * VD) = keep;
+  }
+  if (p.ht) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) *reinterpret_cast<VS*>(p.ht + sbase + i * VD) = s[i];
+  }
+}
+
+// T tokens of the recurrence in fp32, 16 at a time. With S the state before the 16 tokens, a_t the decays,
+// E_tj = a_{j+1} .. a_t and e_t = a_0 .. a_t (products, not exponentials of differences: exact for any decay):
+//   x_t = beta_t (v_t - e_t k_t^T S),  delta_t = x_t - sum_{j<t} beta_t E_tj (k_t . k_j) delta_j,
+//   o_t = e_t q_t^T S + sum_{j<=t} E_tj (q_t . k_j) delta_j,  S' = e_15 S + sum_j k_j E_15,j delta_j:
+// the token-by-token recurrence with its sums in another order, every product in fp32. The contractions over K
+// and over the tokens are v_mfma_f32_16x16x4_f32 (fp32 operands and accumulation, twice the rate of
+// v_fma_f32); the triangular parts are summed in VALU code, where no token reads a later one (a NaN in a token
+// does not reach those before it).
+//   A workgroup owns 64 columns of one (sequence, value head); state waves 0-3 own 16 of them each: S [K x 16]
+// stays in the accumulators (tile a: keys 16a + 4g + r, lane (g, i) column i), which are the B operands of K S
+// and Q S as they stand. Helper waves prepare what does not depend on S, ahead of them: waves 4 and 5 the k and
+// q rows of the tokens two steps ahead (normalised, fp32, in LDS; their loads a step earlier still), wave 6 the
+// decays and the k.k coefficients of the next step, wave 7 its q.k coefficients. One barrier per 16 tokens.
+//   Rounding: the decays' products are formed in 64 bits (by the helpers) and rounded once, a step's update and
+// what earlier tokens take from x are summed apart and added once, and the sums over K run in partial sums, so
+// that the error against 64 bits is that of the token-by-token kernel before it (fp32, 500 tokens of K = 128: o
+// 1.32e-7 against 1.34e-7, state 8.5e-8 against 9.3e-8). 16-bit outputs take two partial sums instead of four: with
+// them the kernel fits 128 registers and two workgroups a CU (16 sequences of 7 tokens 15.3 us against 18.4).
+//   What bounds it: the 3 K / 4 fp32 MFMAs of a step (K = 128: 96 x 32 cycles a wave) and, for few sequences, the
+// chain of a step (K S, x through LDS, the triangular solve, the update). bf16, 16 heads of 128: 16 sequences of 64
+// tokens 37 us against 194 for the kernel before it (a token at a time, two barriers each); fp32, 2 sequences of
+// 512 tokens 122 against 1390; 4 heads of 64, 256 tokens 45 against 384.
+template <typename E, int KD, int VD>
+__global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recurrent_kernel(RecParams p) {
+  constexpr int C = 16, A = KD / 16, KP = KD + 4, P = C + 4;  // 16-byte rows, spread over the banks
+  constexpr int NP = sizeof(E) == 4 ? 4 : 2;
+  __shared__ __align__(16) float kt[3][C * KP], qt[3][C * KP];
+  __shared__ __align__(16) float cm[2][C * P], pm[2][C * P];  // cm[j][t] = beta_t E_tj k_t.k_j, pm[t][j] = E_tj q_t.k_j
+  __shared__ __align__(16) float bs[2][C], es[2][C], ed[2][C];  // beta_t, e_t, E_15,j
+  __shared__ __align__(16) float xs[4][C * P];                  // per state wave: x by column
+  const int t = threadIdx.x, lane = t % kWave, w = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int li = lane % 16, g = lane / 16;
+  constexpr int kSlices = VD / 64;
+  const int hv = blockIdx.x / kSlices;
+  const int64_t n = blockIdx.y;
+  const int h = hv / (int)(p.HV / p.H);
+  int64_t bos, eos;
+  if (p.cu) {
+    bos = load_index(p.cu, p.cu_i32, n);
+    eos = load_index(p.cu, p.cu_i32, n + 1);
+  } else {
+    bos = n * p.T;
+    eos = bos + p.T;
+  }
+  const int steps = (int)((eos - bos + C - 1) / C);
+  auto mm = [](float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); };
+  auto ld4 = [](const float* x) { return *reinterpret_cast<const f32x4*>(x); };
+  auto tok = [&](int i, int c) {  // token c of step i; past the end the last token (its values are cleared)
+    const int64_t at = bos + (int64_t)i * C + c;
+    return at < eos ? at : eos - 1;
+  };
+
+  if (w < 4) {
+    const int col = (blockIdx.x % kSlices) * 64 + w * 16 + li;
+    const int64_t sbase = (n * p.HV + hv) * (int64_t)KD * VD + col;
+    f32x4 s[A];
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[a][r] = p.h0 ? p.h0[sbase + (16 * a + 4 * g + r) * VD] : 0.f;
+    const E* __restrict__ vp = static_cast<const E*>(p.v) + (int64_t)hv * VD + col;
+    E* __restrict__ op = static_cast<E*>(p.o) + (int64_t)hv * VD + col;
+    E vr[4];
+    if (steps > 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vr[r] = vp[tok(0, 4 * g + r) * p.HV * VD];
+    }
+    __syncthreads();
+    __syncthreads();
+    for (int i = 0; i < steps; ++i) {
+      const float* kl = kt[i % 3];
+      const float* ql = qt[i % 3];
+      const int li = opaque_int(lane % 16), g = opaque_int(lane / 16);  // addresses made here, not kept across steps
+      const int b = i & 1, left = (int)(eos - bos - (int64_t)i * C < C ? eos - bos - (int64_t)i * C : C);
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = 4 * g + r < left ? (float)vr[r] : 0.f;
+      if (i + 1 < steps) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vr[r] = vp[tok(i + 1, 4 * g + r) * p.HV * VD];
+      }
+      f32x4 yp[NP]{}, zp[NP]{};  // K S and Q S in partial sums: lane (g, i) column i, tokens 4g + r
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        const f32x4 kf = ld4(kl + li * KP + 16 * a + 4 * g), qf = ld4(ql + li * KP + 16 * a + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          yp[r % NP] = mm(kf[r], s[a][r], yp[r % NP]);
+          zp[r % NP] = mm(qf[r], s[a][r], zp[r % NP]);
+        }
+        if (a % 2) __builtin_amdgcn_sched_barrier(0);  // the rows of two tiles in flight, not of all
+      }
+      f32x4 y = yp[0] + yp[1], z = zp[0] + zp[1];
+      if constexpr (NP == 4) {
+        y += yp[2] + yp[3];
+        z += zp[2] + zp[3];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const f32x4 eg = ld4(es[b] + 4 * g), bg = ld4(bs[b] + 4 * g);
+      f32x4 x[4];  // x, then delta, of this lane's column: all 16 tokens
+      {
+        f32x4 xg;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) xg[r] = 4 * g + r < left ? bg[r] * (v[r] - eg[r] * y[r]) : 0.f;  // y may be 0 * inf
+        *reinterpret_cast<f32x4*>(xs[w] + li * P + 4 * g) = xg;
+        __builtin_amdgcn_wave_barrier();  // the wave reads its own writes (LDS operations of a wave are in order)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = ld4(xs[w] + li * P + 4 * u);
+      }
+      f32x4 sub[4]{};  // what the earlier tokens take from x: summed apart, so that x is rounded once
+#pragma unroll
+      for (int j = 0; j < C; ++j) {
+        x[j / 4][j % 4] -= sub[j / 4][j % 4];  // now delta of token j
+#pragma unroll
+        for (int u = (j + 1) / 4; u < 4; ++u) {
+          const f32x4 c = ld4(cm[b] + j * P + 4 * u);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (4 * u + r > j) sub[u][r] += c[r] * x[j / 4][j % 4];
+        }
+        if (j % 4 == 4 - 1) __builtin_amdgcn_sched_barrier(0);
+      }
+      f32x4 dg;  // delta of the tokens 4g + r
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dg[r] = g < 2 ? (g == 0 ? x[0][r] : x[1][r]) : (g == 2 ? x[2][r] : x[3][r]);
+      const f32x4 edg = ld4(ed[b] + 4 * g);
+      f32x4 db;
+      const float last = es[b][C - 1];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) db[r] = dg[r] * edg[r];
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        f32x4 u{};  // summed apart and added once: one rounding of the state per step
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u = mm(kl[(4 * g + r) * KP + 16 * a + li], db[r], u);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[a][r] = s[a][r] * last + u[r];
+        if (a % 2) __builtin_amdgcn_sched_barrier(0);
+      }
+      f32x4 o{};
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        if (u < g) {  // tokens of earlier quads
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const f32x4 pr = ld4(pm[b] + (4 * g + r) * P + 4 * u);
+            o[r] += (pr[0] * x[u][0] + pr[1] * x[u][1]) + (pr[2] * x[u][2] + pr[3] * x[u][3]);
+          }
+        }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const f32x4 pr = ld4(pm[b] + (4 * g + r) * P + 4 * g);
+#pragma unroll
+        for (int j = 0; j <= r; ++j) o[r] += pr[j] * dg[j];
+        o[r] += eg[r] * z[r];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * g + r < left) op[(bos + (int64_t)i * C + 4 * g + r) * p.HV * VD] = (E)o[r];
+      __syncthreads();
+    }
+    if (p.ht) {
+#pragma unroll
+      for (int a = 0; a < A; ++a)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p.ht[sbase + (16 * a + 4 * g + r) * VD] = s[a][r];
+    }
+  } else if (w < 6) {  // k and q rows: 8 threads per token, KD / 8 elements each
+    constexpr int R = KD / 8;
+    using VK = typename RowVec<E, R>::T;
+    const int row = (t - 256) / 8, pos = (t % 8) * R;
+    const E* __restrict__ kp = static_cast<const E*>(p.k) + (int64_t)h * KD + pos;
+    const E* __restrict__ qp = static_cast<const E*>(p.q) + (int64_t)h * KD + pos;
+    const bool l2 = p.flags & GDN_FLAG_QK_L2NORM;
+    VK kr{}, qr{};
+    auto load = [&](int i) {
+      kr = *reinterpret_cast<const VK*>(kp + tok(i, row) * p.H * KD);
+      qr = *reinterpret_cast<const VK*>(qp + tok(i, row) * p.H * KD);
+    };
+    if (steps > 0) load(0);
+    for (int i = -2; i < steps; ++i) {
+      if (i + 2 < steps) {  // F.normalize: x / max(|x|, 1e-12); q times the scale; zeros past the end
+        const bool live = bos + (int64_t)(i + 2) * C + row < eos;
+        float kf[R], qf[R], kk = 0.f, qq = 0.f;
+#pragma unroll
+        for (int e = 0; e < R; ++e) {
+          kf[e] = live ? (float)kr[e] : 0.f;
+          qf[e] = live ? (float)qr[e] : 0.f;
+          kk += kf[e] * kf[e];
+          qq += qf[e] * qf[e];
+        }
+        float ks = 1.f, qs = p.scale;
+        if (l2) {
+          ks = 1.f / fmaxf(sqrtf(group_sum<8>(kk)), 1e-12f);
+          qs = p.scale / fmaxf(sqrtf(group_sum<8>(qq)), 1e-12f);
+        }
+        float* kl = kt[(i + 2) % 3] + row * KP + pos;
+        float* ql = qt[(i + 2) % 3] + row * KP + pos;
+#pragma unroll
+        for (int e = 0; e < R; e += 4) {
+          *reinterpret_cast<f32x4*>(kl + e) = f32x4{kf[e] * ks, kf[e + 1] * ks, kf[e + 2] * ks, kf[e + 3] * ks};
+          *reinterpret_cast<f32x4*>(ql + e) = f32x4{qf[e] * qs, qf[e + 1] * qs, qf[e + 2] * qs, qf[e + 3] * qs};
+        }
+        if (i + 3 < steps) load(i + 3);
+      }
+      __syncthreads();
+    }
+  } else {  // coefficients of the next step: wave 6 k.k (with beta), wave 7 q.k
+    uint32_t graw = 0, braw = 0;
+    auto load = [&](int i) {
+      graw = load_raw32(p.g, p.dg, tok(i, li) * p.HV + hv);
+      if (w == 6) braw = load_raw32(p.beta, p.db, tok(i, li) * p.HV + hv);
+    };
+    const float neg_a = p.flags & GDN_FLAG_GATE_IN_KERNEL ? -expf(p.A_log[hv]) : 0.f;
+    const float dtb = p.flags & GDN_FLAG_GATE_IN_KERNEL ? p.dt_bias[hv] : 0.f;
+    if (steps > 0) load(0);
+    __syncthreads();
+    for (int i = 0; i <= steps; ++i) {  // step i, while the state waves work on step i - 1
+      if (i < steps) {
+        const int b = i & 1;
+        const bool live = bos + (int64_t)i * C + li < eos;
+        float gv = raw32_to_f32(graw, p.dg), bv = raw32_to_f32(braw, p.db);
+        if (p.flags & GDN_FLAG_GATE_IN_KERNEL) gv = neg_a * softplus_f32(gv + dtb);
+        if (p.flags & GDN_FLAG_BETA_SIGMOID) bv = sigmoid_f32(bv);
+        const double av = live ? exp((double)gv) : 1.0;  // decays in 64 bits up to the products that leave here
+        bv = live ? bv : 0.f;
+        if (i + 1 < steps) load(i + 1);
+        const float* kl = kt[i % 3] + li * KP + 4 * g;
+        const float* rl = w == 6 ? kl : qt[i % 3] + li * KP + 4 * g;
+        f32x4 dp[8]{};  // lane (g, j): rows (tokens) 4g + r, column (earlier token) j
+#pragma unroll
+        for (int a = 0; a < A; a += 2) {
+          const f32x4 k0 = ld4(kl + 16 * a), r0 = ld4(rl + 16 * a), k1 = ld4(kl + 16 * a + 16), r1 = ld4(rl + 16 * a + 16);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            dp[r] = mm(r0[r], k0[r], dp[r]);
+            dp[4 + r] = mm(r1[r], k1[r], dp[4 + r]);
+          }
+          __builtin_amdgcn_sched_barrier(0);  // the rows of two tiles in flight: 128 registers have to do
+        }
+        const int lo = opaque_int(li), go = opaque_int(g);  // compared 32 times: no masks kept across the loop
+        double e = 1.0, ei = 1.0;  // E_mj while m runs; e_t of token li: rounded to fp32 once
+        f32x4 eg{};
+#pragma unroll
+        for (int m = 0; m < C; ++m) {
+          const uint64_t bits = __builtin_bit_cast(uint64_t, av);
+          const double am = __builtin_bit_cast(double, (uint64_t)__builtin_amdgcn_readlane((uint32_t)(bits >> 32), m) << 32 |
+                                                           (uint32_t)__builtin_amdgcn_readlane((uint32_t)bits, m));
+          e *= m > lo ? am : 1.0;
+          if (w == 6) ei *= m <= lo ? am : 1.0;
+          eg[m % 4] = m / 4 == go ? (float)e : eg[m % 4];
+        }
+        const f32x4 d = ((dp[0] + dp[1]) + (dp[2] + dp[3])) + ((dp[4] + dp[5]) + (dp[6] + dp[7]));
+        if (w == 6) {
+          f32x4 c;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float bt = __shfl(bv, 4 * g + r, kWave);
+            c[r] = 4 * g + r > li ? bt * eg[r] * d[r] : 0.f;
+          }
+          *reinterpret_cast<f32x4*>(cm[b] + li * P + 4 * g) = c;
+          if (g == 0) {
+            bs[b][li] = bv;
+            es[b][li] = (float)ei;
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pm[b][(4 * g + r) * P + li] = 4 * g + r >= li ? eg[r] * d[r] : 0.f;
+          if (g == 0) ed[b][li] = (float)e;
+        }
+      }
+      __syncthreads();
     }
   }
-  if (p.ht) store_state<KD, VD>(s, p.ht + sbase);
 }
 
 struct DecodeParams {
@@ -440,12 +779,31 @@ extern "C" int gdn_recurrent_fwd(const void* q, const void* k, const void* v, co
   }
   RecParams p{q, k, v, g, beta, initial_state, o, final_state, cu_seqlens, (flags & GDN_FLAG_CU_INT32) ? 1 : 0,
               T, H, HV, qkv_dtype, g_dtype, beta_dtype, scale, flags, A_log, dt_bias};
-  dim3 grid((unsigned)HV, (unsigned)N), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (K == 128 && V == 128) hipLaunchKernelGGL((gated_delta_recurrent_kernel<128, 128>), grid, block, 0, s, p);
-  else if (K == 64 && V == 64) hipLaunchKernelGGL((gated_delta_recurrent_kernel<64, 64>), grid, block, 0, s, p);
-  else if (K == 128 && V == 64) hipLaunchKernelGGL((gated_delta_recurrent_kernel<128, 64>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((gated_delta_recurrent_kernel<64, 128>), grid, block, 0, s, p);
+  // Few tokens a sequence: the 16-token steps would be mostly padding. bf16, 16 heads of 128, us at 3 / 5 / 8 / 12
+  // tokens in the short kernel and in the 16-token one: 1 sequence 5.9 / 7.5 / 9.3 / 12.0 and 8.5; 16 sequences
+  // 11.1 / 13.8 / 16.6 / 21.7 and 15.3; 64 sequences 27.4 / 32.3 / 40.5 / 55.2 and 42 (heads of 64: 11.3 / 14.8 / 17.8
+  // / 22.8 and 17.5). The line is at 4 tokens, at 6 from 512 waves of 64 columns up and at 8 from 1,024 up, where
+  // the state's bytes set the time of either.
+  const int64_t tokens = cu_seqlens ? T : B * T, cols = N * HV * V;
+  const bool few = tokens <= (cols >= 65536 ? 8 : cols >= 32768 ? 6 : kShortTokens) * N;
+  auto go = [&](auto e_tag, auto k_c, auto v_c) {
+    constexpr int KD = decltype(k_c)::value, VD = decltype(v_c)::value;
+    const dim3 grid((unsigned)(HV * (VD / 64)), (unsigned)N);
+    if (few) hipLaunchKernelGGL((gated_delta_recurrent_short_kernel<decltype(e_tag), KD, VD>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((gated_delta_recurrent_kernel<decltype(e_tag), KD, VD>), grid, dim3(512), 0, s, p);
+  };
+  auto by_dims = [&](auto e_tag) {
+    using C64 = std::integral_constant<int, 64>;
+    using C128 = std::integral_constant<int, 128>;
+    if (K == 128 && V == 128) go(e_tag, C128{}, C128{});
+    else if (K == 64 && V == 64) go(e_tag, C64{}, C64{});
+    else if (K == 128) go(e_tag, C128{}, C64{});
+    else go(e_tag, C64{}, C128{});
+  };
+  if (qkv_dtype == GDN_DTYPE_BF16) by_dims(bf16{});
+  else if (qkv_dtype == GDN_DTYPE_F16) by_dims(f16{});
+  else by_dims(float{});
   return gdn_internal_check_launch("gated_delta_recurrent_kernel");
 }
 

@@ -1,0 +1,93 @@
+"""GPU: the recurrent kernels around their step sizes, against the fp64 oracle.
+
+Lengths around the few-token kernel's 4 tokens and the 16-token steps, sequences of mixed lengths, value heads
+sharing q/k heads, gates that decay to nothing, rows at odd element offsets, and a NaN that must not reach
+earlier tokens, other heads or other sequences. fp32 bound: at most 2^-17 of the largest magnitude (T <= 70
+tokens of K <= 128 products, fp32 sums); 16-bit outputs add half a unit in the last place.
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from oracle import recurrent_gated_delta_rule
+from sorernn_amd import fused_recurrent_gated_delta_rule
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+HALF_ULP = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 2.0**-24}
+
+
+def _inputs(b, t, h, hv, kd, vd, n, dtype, seed):
+    gen = torch.Generator().manual_seed(seed)
+    q, k = (F.normalize(torch.randn(b, t, h, kd, generator=gen), dim=-1).to(dtype) for _ in range(2))
+    v = torch.randn(b, t, hv, vd, generator=gen).to(dtype)
+    g = -F.softplus(torch.randn(b, t, hv, generator=gen)) * (torch.rand(b, t, hv, generator=gen) * 6 - 4).exp()
+    g[torch.rand(b, t, hv, generator=gen) < 0.05] = -float("inf")  # a token that forgets everything
+    g[torch.rand(b, t, hv, generator=gen) < 0.05] = -300.0
+    beta = torch.randn(b, t, hv, generator=gen).sigmoid()
+    return q, k, v, g, beta, torch.randn(n, hv, kd, vd, generator=gen)
+
+
+def _check(o, st, o_ref, st_ref, dtype):
+    err, top = (o.double().cpu() - o_ref).abs(), o_ref.abs().max().item()
+    bound = 2.0**-17 * top + HALF_ULP[dtype] * o_ref.abs() * 1.01
+    assert (err <= bound).all(), f"o: {(err / bound).max().item():.2f} of the bound"
+    assert ((st.double().cpu() - st_ref).abs() <= 2.0**-17 * st_ref.abs().max()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("t", [1, 3, 4, 5, 8, 15, 16, 17, 33, 70])
+@pytest.mark.parametrize("b,h,hv,kd,vd", [(2, 2, 4, 128, 128), (1, 3, 3, 64, 128), (3, 1, 2, 128, 64), (1, 2, 2, 64, 64)])
+def test_lengths_around_the_steps(b, h, hv, kd, vd, t, dtype):
+    q, k, v, g, beta, h0 = _inputs(b, t, h, hv, kd, vd, b, dtype, 10 * t + b)
+    o, st = fused_recurrent_gated_delta_rule(*(x.to(DEV) for x in (q, k, v, g, beta)), initial_state=h0.to(DEV),
+                                             output_final_state=True)
+    o_ref, st_ref = recurrent_gated_delta_rule(*(x.double() for x in (q, k, v, g, beta)), kd**-0.5, h0.double(), True)
+    _check(o, st, o_ref.double(), st_ref.double(), dtype)
+
+
+@pytest.mark.parametrize("lens", [[1, 2, 1, 4], [1, 40, 3, 16, 17, 1], [5, 5, 2, 1]])
+def test_mixed_lengths_with_norm_and_gate_in_kernel(lens):
+    t, n = sum(lens), len(lens)
+    q, k, v, _, _, h0 = _inputs(1, t, 2, 4, 128, 128, n, torch.bfloat16, t)
+    gen = torch.Generator().manual_seed(t)
+    q, k = (3 * torch.randn(q.shape, generator=gen)).bfloat16(), (3 * torch.randn(k.shape, generator=gen)).bfloat16()
+    k[0, t // 2] = 0  # a zero row: 0 / max(0, 1e-12)
+    a, bl = (torch.randn(1, t, 4, generator=gen).bfloat16() for _ in range(2))
+    a_log, dtb = torch.rand(4, generator=gen) * 2, torch.randn(4, generator=gen)
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()])
+    o, st = fused_recurrent_gated_delta_rule(
+        *(x.to(DEV) for x in (q, k, v, a, bl)), initial_state=h0.to(DEV), output_final_state=True, cu_seqlens=cu.to(DEV),
+        cu_seqlens_cpu=cu, use_qk_l2norm_in_kernel=True, use_beta_sigmoid_in_kernel=True, use_gate_in_kernel=True,
+        A_log=a_log.to(DEV), dt_bias=dtb.to(DEV))
+    g = -a_log.double().exp() * F.softplus(a.double() + dtb.double())
+    o_ref, st_ref = recurrent_gated_delta_rule(F.normalize(q.double(), dim=-1), F.normalize(k.double(), dim=-1), v.double(), g,
+                                               bl.double().sigmoid(), 128**-0.5, h0.double(), True, cu_seqlens=cu)
+    _check(o, st, o_ref.double(), st_ref.double(), torch.bfloat16)
+
+
+@pytest.mark.parametrize("t", [3, 37])
+def test_rows_at_odd_element_offsets(t):
+    q, k, v, g, beta, h0 = _inputs(1, t, 2, 2, 128, 128, 1, torch.bfloat16, t)
+
+    def odd(x):  # the same values, contiguous, one element into a larger allocation
+        flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=DEV)
+        flat[1:] = x.flatten().to(DEV)
+        return flat[1:].view(x.shape)
+
+    o, st = fused_recurrent_gated_delta_rule(*(odd(x) for x in (q, k, v, g, beta)), initial_state=odd(h0), output_final_state=True)
+    o_ref, st_ref = recurrent_gated_delta_rule(*(x.double() for x in (q, k, v, g, beta)), 128**-0.5, h0.double(), True)
+    _check(o, st, o_ref.double(), st_ref.double(), torch.bfloat16)
+
+
+@pytest.mark.parametrize("t,bad", [(4, 2), (40, 21), (16, 15)])
+@pytest.mark.parametrize("where", ["q", "k", "v", "g", "beta"])
+def test_nan_reaches_only_later_tokens_of_its_head(t, bad, where):
+    x = dict(zip(("q", "k", "v", "g", "beta"), _inputs(2, t, 2, 2, 64, 64, 2, torch.float32, t)[:5]))
+    x[where][0, bad, 1] = float("nan")
+    o, st = fused_recurrent_gated_delta_rule(*(x[n].to(DEV) for n in ("q", "k", "v", "g", "beta")), output_final_state=True)
+    assert torch.isfinite(o[0, :bad]).all() and torch.isfinite(o[:, :, 0]).all() and torch.isfinite(o[1]).all()
+    assert torch.isfinite(st[1]).all() and torch.isfinite(st[0, 0]).all()
+    assert not torch.isfinite(o[0, bad, 1]).any()
+    if where == "q":
+        assert torch.isfinite(o[0, bad + 1:]).all() and torch.isfinite(st).all()
