@@ -655,11 +655,13 @@ __global__ __launch_bounds__(kNT, 1) void gated_delta_chunk_kernel(ChunkParams p
 #pragma unroll
     for (int u = 0; u < QKPT; ++u) dst[u] = buf_load16(rs, base + (uint32_t)(u * (256 / KCH)) * qk_row);
   };
-  auto stage_rows = [&](const bf16x8 (&src)[QKPT], f16* dst, int tq) {  // bf16 rows (L2-normalised when asked) -> fp16
+  // bf16 rows (L2-normalised when asked, the tile's QKPT rows per lane side by side) -> fp16
+  auto stage_rows = [&](bf16x8 (&src)[QKPT], f16* dst, int tq) {
+    if (l2) l2norm_row_chunks<KCH>(src);
     f16* const d0 = dst + (tq / KCH) * KP + (((tq % KCH) ^ kq_sw(tq / KCH)) << 3);  // rows tq/KCH + 16u: same swizzle
 #pragma unroll
     for (int u = 0; u < QKPT; ++u)
-      *reinterpret_cast<f16x8*>(d0 + u * (256 / KCH) * KP) = bf16_to_f16x8(l2 ? l2norm_row_chunk<KCH>(src[u]) : src[u]);
+      *reinterpret_cast<f16x8*>(d0 + u * (256 / KCH) * KP) = bf16_to_f16x8(src[u]);
   };
   // Thread tq of waves 4-5: T - I chunks tq + 128u (row tq / 8 + 16u, 8 chunks of 16 B per row)
   // and V-slice chunks tq + 128u (row tq / 4 + 32u, 4 chunks per row).

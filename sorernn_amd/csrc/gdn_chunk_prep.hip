@@ -131,9 +131,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(3))) __launch_bounds__(kWave) void
         v[s] = ss;
       }
 #pragma unroll
-      for (int s = 0; s < KS; ++s) v[s] += __shfl_xor(v[s], 16, kWave);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) v[s] += __shfl_xor(v[s], 32, kWave);
+      for (int s = 0; s < KS; ++s) v[s] = xor32_sum(xor16_sum(v[s]));
       float tot;
       if constexpr (KS == 4) tot = (v[0] + v[1]) + (v[2] + v[3]);
       else tot = v[0] + v[1];

@@ -96,6 +96,16 @@ __device__ __forceinline__ float dpp_add(float v) {
   return v + __int_as_float(s);
 }
 
+// x + (x of the lane 16, or 32, away): gfx950's 16- and 32-lane swaps, in the VALU.
+__device__ __forceinline__ float xor16_sum(float x) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float xor32_sum(float x) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Sum over aligned groups of N lanes (N = 8, 16 or 32) with DPP: quad_perm [1,0,3,2] and [2,3,0,1]
 // (0xb1, 0x4e), row_half_mirror (0x141, pairs the two quads of an 8-lane half) and row_mirror
 // (0x140, pairs the two halves of a 16-lane row), then gfx950's 16-lane swap of row pairs. Every
@@ -107,10 +117,7 @@ __device__ __forceinline__ float group_sum(float x) {
   x = dpp_add<0x4e, 0xf>(x);
   x = dpp_add<0x141, 0xf>(x);
   if (N >= 16) x = dpp_add<0x140, 0xf>(x);
-  if (N == 32) {
-    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
+  if (N == 32) x = xor16_sum(x);
   return x;
 }
 

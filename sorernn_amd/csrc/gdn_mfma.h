@@ -172,20 +172,35 @@ __device__ __forceinline__ void chunk_gates_from_raw(ChunkGates& gs, uint32_t gr
   gs.dlast[lane] = __expf(last - cs);
 }
 
-// F.normalize over a q/k row held by KCH consecutive lanes (8 bf16 each), rounded back to bf16.
-// 1 / max(||x||, 1e-12) as v_rsq_f32 of max(||x||^2, 1e-24): about 1 ulp of fp32 from the IEEE
+// F.normalize over q/k rows, each held by KCH consecutive lanes (8 bf16 each), rounded back to bf16; U rows
+// per lane. 1 / max(||x||, 1e-12) as v_rsq_f32 of max(||x||^2, 1e-24): about 1 ulp of fp32 from the IEEE
 // sqrt and divide, far below the bf16 rounding that follows, and a few instructions instead of the
-// IEEE sequences (this runs on the helper waves once per 16-byte chunk of every q/k row).
+// IEEE sequences (this runs on the helper waves once per 16-byte chunk of every q/k row). The U rows' sums
+// advance side by side: one row alone is a chain of 8 dependent additions, 4 DPP steps with their wait
+// states and the reciprocal root.
+template <int KCH, int U>
+__device__ __forceinline__ void l2norm_row_chunks(bf16x8 (&x)[U]) {
+  float ss[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) ss[u] = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int u = 0; u < U; ++u) ss[u] += (float)x[u][i] * (float)x[u][i];
+#pragma unroll
+  for (int u = 0; u < U; ++u) ss[u] = group_sum<KCH>(ss[u]);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float inv = __builtin_amdgcn_rsqf(fmaxf(ss[u], 1e-24f));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[u][i] = static_cast<bf16>((float)x[u][i] * inv);
+  }
+}
 template <int KCH>
 __device__ __forceinline__ bf16x8 l2norm_row_chunk(bf16x8 x) {
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ss += (float)x[i] * (float)x[i];
-  ss = group_sum<KCH>(ss);
-  const float inv = __builtin_amdgcn_rsqf(fmaxf(ss, 1e-24f));
-#pragma unroll
-  for (int i = 0; i < 8; ++i) x[i] = static_cast<bf16>((float)x[i] * inv);
-  return x;
+  bf16x8 r[1] = {x};
+  l2norm_row_chunks<KCH>(r);
+  return r[0];
 }
 
 }  // namespace gdn
