@@ -243,6 +243,10 @@ GDN_API int gdn_causal_conv1d_fwd(const void* x, const float* weight, const floa
  */
 GDN_API int gdn_l2norm_fwd(const void* x, void* y, int64_t rows, int64_t D, int dtype, float eps, void* stream);
 
+/* gdn_l2norm_fwd of q and of k (the same number of rows each) in one launch. */
+GDN_API int gdn_qk_l2norm_fwd(const void* q, const void* k, void* q_out, void* k_out, int64_t rows, int64_t D, int dtype,
+                              float eps, void* stream);
+
 /*
  * Gated RMSNorm: y = x * rsqrt(mean(x^2) + eps) * weight (+ bias) * act(gate), per row of D.
  * Replaces FLA rms_norm_gated(o, gate, weight, None, activation="swish", eps) at

@@ -21,11 +21,17 @@ struct NormParams {
   float eps;
   int mode;   // 0 = L2 norm, 1 = (gated) RMSNorm
   int split;  // RMSNorm with a gate: the norm (w, bias) and act(gate) each rounded before their product
+  const void* x2;  // a second tensor of the same rows, normalised by the blocks with blockIdx.y = 1
+  void* y2;
 };
 
 constexpr int kNormMaxPerLane = 16;  // D <= 1024
 
 __global__ __launch_bounds__(256) void gated_delta_norm_kernel(NormParams p) {
+  if (blockIdx.y) {
+    p.x = p.x2;
+    p.y = p.y2;
+  }
   const int lane = threadIdx.x % kWave;
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) / kWave;
@@ -72,6 +78,10 @@ constexpr int kNormV8Groups = 4;
 
 template <typename E, int LPR>
 __global__ __launch_bounds__(256) void gated_delta_norm_v8_kernel(NormParams p) {
+  if (blockIdx.y) {
+    p.x = p.x2;
+    p.y = p.y2;
+  }
   typedef E V8 __attribute__((ext_vector_type(8)));
   constexpr int RPW = kWave / LPR, U = kNormV8Groups;
   const int lane = threadIdx.x % kWave, sub = lane / LPR, li = lane % LPR;
@@ -400,12 +410,14 @@ static int launch_norm(const NormParams& p, void* stream, const char* what) {
   if (p.rows == 0) return GDN_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool aligned = ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.y) |
+                         reinterpret_cast<uintptr_t>(p.x2) | reinterpret_cast<uintptr_t>(p.y2) |
                          reinterpret_cast<uintptr_t>(p.gate)) & 15) == 0;
+  const unsigned two = p.x2 ? 2 : 1;
   if (aligned && (p.D == 64 || p.D == 128) && (p.dt == GDN_DTYPE_BF16 || p.dt == GDN_DTYPE_F16)) {
     const int64_t rpb = 4 * (kWave / (p.D / 8)) * kNormV8Groups;  // rows per 256-thread block and pass
     int64_t vb = (p.rows + rpb - 1) / rpb;
     if (vb > 65536) vb = 65536;
-    const dim3 g((unsigned)vb), b(256);
+    const dim3 g((unsigned)vb, two), b(256);
     if (p.dt == GDN_DTYPE_BF16) {
       if (p.D == 128) hipLaunchKernelGGL((gated_delta_norm_v8_kernel<bf16, 16>), g, b, 0, s, p);
       else hipLaunchKernelGGL((gated_delta_norm_v8_kernel<bf16, 8>), g, b, 0, s, p);
@@ -417,7 +429,7 @@ static int launch_norm(const NormParams& p, void* stream, const char* what) {
   }
   int64_t blocks = (p.rows + 3) / 4;
   if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL(gated_delta_norm_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(gated_delta_norm_kernel, dim3((unsigned)blocks, two), dim3(256), 0, s, p);
   return gdn_internal_check_launch(what);
 }
 
@@ -427,7 +439,7 @@ using namespace gdn;
 
 int gdn::gdn_internal_rms_norm_gated(const void* x, const void* gate, const float* w, void* y, int64_t rows, int64_t D,
                                      float eps, int split, hipStream_t s) {
-  NormParams p{x, gate, w, nullptr, y, rows, D, GDN_DTYPE_BF16, GDN_ACT_SILU, eps, 1, split};
+  NormParams p{x, gate, w, nullptr, y, rows, D, GDN_DTYPE_BF16, GDN_ACT_SILU, eps, 1, split, nullptr, nullptr};
   return launch_norm(p, s, "gated_delta_norm_kernel(rms)");
 }
 
@@ -440,8 +452,22 @@ extern "C" int gdn_l2norm_fwd(const void* x, void* y, int64_t rows, int64_t D, i
     gdn_internal_set_error("gdn_l2norm_fwd: D=%lld exceeds %d", (long long)D, kNormMaxPerLane * kWave);
     return GDN_ERR_UNSUPPORTED;
   }
-  NormParams p{x, nullptr, nullptr, nullptr, y, rows, D, dtype, GDN_ACT_NONE, eps, 0};
+  NormParams p{x, nullptr, nullptr, nullptr, y, rows, D, dtype, GDN_ACT_NONE, eps, 0, 0, nullptr, nullptr};
   return launch_norm(p, stream, "gated_delta_norm_kernel(l2)");
+}
+
+extern "C" int gdn_qk_l2norm_fwd(const void* q, const void* k, void* q_out, void* k_out, int64_t rows, int64_t D, int dtype,
+                                 float eps, void* stream) {
+  if (!q || !k || !q_out || !k_out || rows < 0 || D <= 0) {
+    gdn_internal_set_error("gdn_qk_l2norm_fwd: bad arguments (rows=%lld D=%lld)", (long long)rows, (long long)D);
+    return GDN_ERR_INVALID;
+  }
+  if (D > kNormMaxPerLane * kWave) {
+    gdn_internal_set_error("gdn_qk_l2norm_fwd: D=%lld exceeds %d", (long long)D, kNormMaxPerLane * kWave);
+    return GDN_ERR_UNSUPPORTED;
+  }
+  NormParams p{q, nullptr, nullptr, nullptr, q_out, rows, D, dtype, GDN_ACT_NONE, eps, 0, 0, k, k_out};
+  return launch_norm(p, stream, "gated_delta_norm_kernel(qk l2)");
 }
 
 extern "C" int gdn_rms_norm_gated_fwd(const void* x, const void* gate, const float* weight, const float* bias, void* y,
@@ -458,7 +484,7 @@ extern "C" int gdn_rms_norm_gated_fwd(const void* x, const void* gate, const flo
     gdn_internal_set_error("gdn_rms_norm_gated_fwd: unknown activation %d", activation);
     return GDN_ERR_INVALID;
   }
-  NormParams p{x, gate, weight, bias, y, rows, D, dtype, activation, eps, 1};
+  NormParams p{x, gate, weight, bias, y, rows, D, dtype, activation, eps, 1, 0, nullptr, nullptr};
   return launch_norm(p, stream, "gated_delta_norm_kernel(rms)");
 }
 

@@ -176,7 +176,7 @@ def _gdn_call(entry, name, q, k, v, g, beta, scale, initial_state, output_final_
     q_raw, k_raw = q, k
     if (entry == "gdn_chunk_fwd" and (flags & _lib.FLAG_QK_L2NORM) and not needs_grad
             and _l2norm_first(q, n, hv, vd, b * t)):
-        q, k = (_l2norm_rows(x) for x in (q, k))
+        q, k = _l2norm_qk(q, k)
         flags &= ~_lib.FLAG_QK_L2NORM
     if entry == "gdn_chunk_fwd":
         # the torch.library op (sorernn::chunk_gated_delta_rule_fwd): traceable by torch.compile, with
@@ -334,7 +334,7 @@ def chunk_gated_delta_rule_gated_norm(
     word = _range.before_call(q.device)
     q_raw, k_raw = q, k
     if (flags & _lib.FLAG_QK_L2NORM) and _l2norm_first(q, n, hv, vd, b * t):
-        q, k = (_l2norm_rows(x) for x in (q, k))
+        q, k = _l2norm_qk(q, k)
         flags &= ~_lib.FLAG_QK_L2NORM
     q, k, v, g, beta, gate = (x.contiguous() for x in (q, k, v, g, beta, gate))
     w = norm_weight.float().contiguous()
@@ -577,29 +577,35 @@ def _l2norm_first(q: Tensor, n: int, hv: int, vd: int, tokens: int) -> bool:
     before the chunk kernels (which then run without the flag) instead of inside them.
 
     Inside, each of a chain's V/32 state-kernel workgroups normalises the chain's q/k rows on the
-    helper waves that set the step time, ~0.9 us more per chunk step. The row kernel instead costs a
-    pass over q and k (read and write) on the whole chip. That pays when the state kernel leaves
-    half the CUs or more idle and its chains are long. Measured per call (HIP events): B=2, T=8192,
-    16 heads of 128 (32 chains, 128 workgroups): 243 us against 310 us; B=4, T=4096 (256
-    workgroups): 180 us against 170 us, so the flag stays in the kernels there."""
+    helper waves that set the step time: ~0.9 us more per 64-token step at K = 128 (0.35 at 64; 0.6 where several
+    chains follow one another on a CU). The row kernel instead costs a pass over q and k (read and write, 5.2 TB/s)
+    and a launch, ~3 us. First, when that saves 4 us (the call's host work grows by about as much). Measured per
+    call in the kernels / first, 16 heads of 128: 1 x 512 tokens 32.4 / 34.7 us, 1 x 1000 49.7 / 41.6, 2 x 4096
+    161 / 125, 3 x 4096 165 / 149, 4 x 4096 172 / 176, 1 x 16384 589 / 380; of 64: 1 x 1000 32.8 / 34.1, 2 x 4096
+    98 / 89, 4 x 2048 57.7 / 59.5."""
     dev = q.get_device()
     cus = _cu_count.get(dev)
     if cus is None:
         cus = _cu_count[dev] = torch.cuda.get_device_properties(dev).multi_processor_count
-    return 2 * n * hv * max(1, vd // 32) <= cus and tokens >= 2048 * n
+    kd = q.shape[3]
+    rounds = n * hv * max(1, vd // 32) / cus
+    per_step = 0.6 if rounds > 1 else 0.9 if kd >= 128 else 0.35
+    saved = per_step * tokens / (64 * max(1, n)) * max(1.0, rounds)
+    return saved > 3 + 8 * tokens * hv * kd / 5.2e6 + 4  # hv: q/k heads are at most as many
 
 
-def _l2norm_rows(x: Tensor, eps: float = 1e-12) -> Tensor:
-    """``l2norm`` without grad: plain eager calls go to the kernel directly (no dispatcher round trip)."""
-    if not _plain_eager(x):
-        return _library.l2norm_fwd(x, float(eps))
-    xc = x.contiguous()
-    y = torch.empty_like(xc)
-    d = xc.shape[-1]
-    if xc.numel():
-        _lib.call("gdn_l2norm_fwd", _lib.ptr(xc), _lib.ptr(y), xc.numel() // d, d, _lib.dtype_code(xc.dtype), float(eps),
-                  _lib.stream_of(xc))
-    return y
+def _l2norm_qk(q: Tensor, k: Tensor, eps: float = 1e-12) -> tuple[Tensor, Tensor]:
+    """``l2norm`` of q and k without grad: plain eager calls go to the kernel directly (one launch for both, no
+    dispatcher round trip)."""
+    if not _plain_eager(q):
+        return _library.l2norm_fwd(q, float(eps)), _library.l2norm_fwd(k, float(eps))
+    q, k = q.contiguous(), k.contiguous()
+    qn, kn = torch.empty_like(q), torch.empty_like(k)
+    d = q.shape[-1]
+    if q.numel():
+        _lib.call("gdn_qk_l2norm_fwd", q.data_ptr(), k.data_ptr(), qn.data_ptr(), kn.data_ptr(), q.numel() // d, d,
+                  _lib.dtype_code(q.dtype), float(eps), _lib.stream_of(q))
+    return qn, kn
 
 
 def l2norm(x: Tensor, eps: float = 1e-12) -> Tensor:
