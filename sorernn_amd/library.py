@@ -19,10 +19,67 @@ from typing import Optional
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
+from torch.autograd.function import once_differentiable
 
 from sorernn_amd import _lib
 
 C = 64  # chunk length
+
+
+def plain_eager(*tensors) -> bool:
+    """True when nothing but the autograd engine looks at these tensors' operators: ordinary tensors, no
+    compile or FX tracing, no dispatch mode, no functorch transform (vmap, grad, jvp), no forward-mode level."""
+    if torch.compiler.is_compiling():
+        return False
+    return (all(t is None or type(t) is Tensor or type(t) is torch.nn.Parameter for t in tensors)
+            and not torch.fx._symbolic_trace._is_fx_tracing_flag
+            and torch.utils._python_dispatch._get_current_dispatch_mode() is None
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and forward_ad._current_level < 0)
+
+
+def _eager_function(impl, setup, backward):
+    """The autograd function of an op for plain eager calls: the op's implementation, context and formula without
+    the dispatcher and the custom-op wrappers, which cost the host more per call than the kernels run (a conv
+    forward and backward of 4,096 x 2,048 tokens takes 40 us on the GPU, its host work took 160 us and takes 100). Saved tensors go through
+    ``save_for_backward`` as there (hooks see them); a second derivative raises, as there."""
+
+    class EagerOp(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, *args):
+            out = impl(*args)
+            setup(ctx, args, out)
+            if isinstance(out, tuple):
+                ctx.mark_non_differentiable(*(t for t in out if not t.dtype.is_floating_point))
+            return out
+
+        @staticmethod
+        @once_differentiable
+        def backward(ctx, *grads):
+            return backward(ctx, *grads)
+
+    return EagerOp.apply
+
+
+def _eager(op, impl, function, *args):
+    """Runs ``op``: through the dispatcher where anything may look at it, else directly, with ``function`` under grad."""
+    if torch.compiler.is_compiling():
+        return op(*args)
+    tensors = [a for a in args if isinstance(a, Tensor)]
+    if not plain_eager(*tensors):
+        return op(*args)
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return function(*args)
+    return impl(*args)
+
+
+def _run_bwd(op, impl, *args):
+    """A backward op: directly in an ordinary backward pass; with ``create_graph`` through the op, whose outputs
+    then refuse a second derivative."""
+    if not torch.is_grad_enabled() and plain_eager(*(a for a in args if isinstance(a, Tensor))):
+        return impl(*args)
+    return op(*args)
 
 
 def _align256(x):
@@ -91,8 +148,8 @@ def chunk_fwd_impl(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, ini
     return o, final, states, ws
 
 
-# The registered op; ``chunk_fwd_impl`` is its implementation, which the eager inference path of
-# ``ops.py`` calls directly (no dispatcher round trip when nothing traces, records or differentiates).
+# The registered op; ``chunk_fwd_impl`` is its implementation, which plain eager calls run directly
+# (``chunk_fwd_call``: no dispatcher round trip when nothing traces or records).
 chunk_fwd = torch.library.custom_op("sorernn::chunk_gated_delta_rule_fwd", mutates_args=())(chunk_fwd_impl)
 
 
@@ -109,11 +166,10 @@ def _chunk_fwd_fake(q, k, v, g, beta, initial_state, A_log, dt_bias, cu_seqlens,
     return o, final, states, ws
 
 
-@torch.library.custom_op("sorernn::chunk_gated_delta_rule_bwd", mutates_args=())
-def chunk_bwd(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, d_o: Tensor, d_final_state: Optional[Tensor],
-              chunk_states: Tensor, fwd_workspace: Tensor, A_log: Optional[Tensor], dt_bias: Optional[Tensor],
-              cu_seqlens: Optional[Tensor], scale: float, flags: int, num_seqs: int,
-              initial_state_grad: bool) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
+def chunk_bwd_impl(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, d_o: Tensor, d_final_state: Optional[Tensor],
+                   chunk_states: Tensor, fwd_workspace: Tensor, A_log: Optional[Tensor], dt_bias: Optional[Tensor],
+                   cu_seqlens: Optional[Tensor], scale: float, flags: int, num_seqs: int,
+                   initial_state_grad: bool) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     b, t, h, kd = q.shape
     hv, vd = v.shape[2], v.shape[3]
     n = num_seqs
@@ -145,6 +201,9 @@ def chunk_bwd(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, d_o: Ten
         dal.zero_()
         ddt.zero_()
     return dq, dk, dv, dg, db, dh0, dal, ddt
+
+
+chunk_bwd = torch.library.custom_op("sorernn::chunk_gated_delta_rule_bwd", mutates_args=())(chunk_bwd_impl)
 
 
 @chunk_bwd.register_fake
@@ -179,7 +238,7 @@ def _backward(ctx, d_o, d_final, _d_states, _d_ws):
     if d_final is not None and d_final.numel() == 0:
         d_final = None
     want_h0 = ctx.h0_dtype is not None and ctx.needs_input_grad[5]
-    dq, dk, dv, dg, db, dh0, dal, ddt = chunk_bwd(q, k, v, g, beta, d_o, d_final, states, ws, A_log, dt_bias,
+    dq, dk, dv, dg, db, dh0, dal, ddt = _run_bwd(chunk_bwd, chunk_bwd_impl, q, k, v, g, beta, d_o, d_final, states, ws, A_log, dt_bias,
                                                   cu_seqlens, scale, flags, num_seqs, want_h0)
     gate = bool(flags & _lib.FLAG_GATE_IN_KERNEL)
     return (dq, dk, dv, dg, db, dh0.to(ctx.h0_dtype) if want_h0 else None,
@@ -188,15 +247,20 @@ def _backward(ctx, d_o, d_final, _d_states, _d_ws):
 
 
 chunk_fwd.register_autograd(_backward, setup_context=_setup_context)
+_chunk_fwd_eager = _eager_function(chunk_fwd_impl, _setup_context, _backward)
+
+
+def chunk_fwd_call(*args):
+    """``chunk_fwd`` as the Python entry points call it: directly when nothing traces or records."""
+    return _eager(chunk_fwd, chunk_fwd_impl, _chunk_fwd_eager, *args)
 
 
 # ---------------------------------------------------------------------------------------------------
 # causal conv1d (+ SiLU): sorernn::causal_conv1d_fwd / _bwd
 # ---------------------------------------------------------------------------------------------------
-@torch.library.custom_op("sorernn::causal_conv1d_fwd", mutates_args=())
-def conv_fwd(x: Tensor, weight: Tensor, bias: Optional[Tensor], initial_state: Optional[Tensor],
-             cu_seqlens: Optional[Tensor], activation: int, flags: int, num_seqs: int,
-             output_final_state: bool) -> tuple[Tensor, Tensor]:
+def conv_fwd_impl(x: Tensor, weight: Tensor, bias: Optional[Tensor], initial_state: Optional[Tensor],
+                  cu_seqlens: Optional[Tensor], activation: int, flags: int, num_seqs: int,
+                  output_final_state: bool) -> tuple[Tensor, Tensor]:
     b, t, c = x.shape
     w = weight.shape[1]
     xc = x.contiguous()
@@ -212,16 +276,18 @@ def conv_fwd(x: Tensor, weight: Tensor, bias: Optional[Tensor], initial_state: O
     return y, fin
 
 
+conv_fwd = torch.library.custom_op("sorernn::causal_conv1d_fwd", mutates_args=())(conv_fwd_impl)
+
+
 @conv_fwd.register_fake
 def _conv_fwd_fake(x, weight, bias, initial_state, cu_seqlens, activation, flags, num_seqs, output_final_state):
     c, w = x.shape[2], weight.shape[1]
     return torch.empty_like(x), x.new_empty((num_seqs, c, w) if output_final_state else (0,))
 
 
-@torch.library.custom_op("sorernn::causal_conv1d_bwd", mutates_args=())
-def conv_bwd(x: Tensor, weight: Tensor, bias: Optional[Tensor], initial_state: Optional[Tensor],
-             cu_seqlens: Optional[Tensor], dy: Tensor, activation: int, flags: int,
-             num_seqs: int) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+def conv_bwd_impl(x: Tensor, weight: Tensor, bias: Optional[Tensor], initial_state: Optional[Tensor],
+                  cu_seqlens: Optional[Tensor], dy: Tensor, activation: int, flags: int,
+                  num_seqs: int) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     b, t, c = x.shape
     w = weight.shape[1]
     xc = x.contiguous()
@@ -241,6 +307,9 @@ def conv_bwd(x: Tensor, weight: Tensor, bias: Optional[Tensor], initial_state: O
               _lib.ptr(dw), _lib.ptr(db if bias is not None else None),
               _lib.ptr(dinit if initial_state is not None else None), _lib.ptr(ws), ws.numel(), _lib.stream_of(xc))
     return dx, dw, db, dinit
+
+
+conv_bwd = torch.library.custom_op("sorernn::causal_conv1d_bwd", mutates_args=())(conv_bwd_impl)
 
 
 @conv_bwd.register_fake
@@ -265,19 +334,25 @@ def _conv_backward(ctx, dy, dfin):
     activation, flags, num_seqs = ctx.meta
     if dy is None:
         dy = torch.zeros_like(x)
-    dx, dw, db, dinit = conv_bwd(x, weight, bias, initial_state, cu_seqlens, dy, activation, flags, num_seqs)
+    dx, dw, db, dinit = _run_bwd(conv_bwd, conv_bwd_impl, x, weight, bias, initial_state, cu_seqlens, dy, activation, flags,
+                                 num_seqs)
     return (dx, dw.to(weight.dtype), None if bias is None else db.to(bias.dtype),
             None if initial_state is None else dinit.to(initial_state.dtype), None, None, None, None, None)
 
 
 conv_fwd.register_autograd(_conv_backward, setup_context=_conv_setup)
+_conv_fwd_eager = _eager_function(conv_fwd_impl, _conv_setup, _conv_backward)
+
+
+def conv_fwd_call(*args):
+    """``conv_fwd`` as the Python entry points call it: directly when nothing traces or records."""
+    return _eager(conv_fwd, conv_fwd_impl, _conv_fwd_eager, *args)
 
 
 # ---------------------------------------------------------------------------------------------------
 # L2 norm and gated RMSNorm: sorernn::l2norm_fwd / _bwd, sorernn::rms_norm_gated_fwd / _bwd
 # ---------------------------------------------------------------------------------------------------
-@torch.library.custom_op("sorernn::l2norm_fwd", mutates_args=())
-def l2norm_fwd(x: Tensor, eps: float) -> Tensor:
+def l2norm_fwd_impl(x: Tensor, eps: float) -> Tensor:
     xc = x.contiguous()
     y = torch.empty_like(xc)
     d = xc.shape[-1]
@@ -286,13 +361,15 @@ def l2norm_fwd(x: Tensor, eps: float) -> Tensor:
     return y
 
 
+l2norm_fwd = torch.library.custom_op("sorernn::l2norm_fwd", mutates_args=())(l2norm_fwd_impl)
+
+
 @l2norm_fwd.register_fake
 def _l2norm_fwd_fake(x, eps):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("sorernn::l2norm_bwd", mutates_args=())
-def l2norm_bwd(x: Tensor, dy: Tensor, eps: float) -> Tensor:
+def l2norm_bwd_impl(x: Tensor, dy: Tensor, eps: float) -> Tensor:
     xc = x.contiguous()
     dyc = dy.to(x.dtype).contiguous()
     dx = torch.empty_like(xc)
@@ -300,6 +377,9 @@ def l2norm_bwd(x: Tensor, dy: Tensor, eps: float) -> Tensor:
     _lib.call("gdn_l2norm_bwd", _lib.ptr(xc), _lib.ptr(dyc), _lib.ptr(dx), xc.numel() // max(d, 1), d,
               _lib.dtype_code(xc.dtype), eps, _lib.stream_of(xc))
     return dx
+
+
+l2norm_bwd = torch.library.custom_op("sorernn::l2norm_bwd", mutates_args=())(l2norm_bwd_impl)
 
 
 @l2norm_bwd.register_fake
@@ -314,15 +394,20 @@ def _l2_setup(ctx, inputs, output):
 
 def _l2_backward(ctx, dy):
     (x,) = ctx.saved_tensors
-    return l2norm_bwd(x, dy, ctx.eps), None
+    return _run_bwd(l2norm_bwd, l2norm_bwd_impl, x, dy, ctx.eps), None
 
 
 l2norm_fwd.register_autograd(_l2_backward, setup_context=_l2_setup)
+_l2norm_fwd_eager = _eager_function(l2norm_fwd_impl, _l2_setup, _l2_backward)
 
 
-@torch.library.custom_op("sorernn::rms_norm_gated_fwd", mutates_args=())
-def rms_fwd(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], bias: Optional[Tensor], eps: float,
-            activation: int) -> Tensor:
+def l2norm_fwd_call(*args):
+    """``l2norm_fwd`` as the Python entry points call it: directly when nothing traces or records."""
+    return _eager(l2norm_fwd, l2norm_fwd_impl, _l2norm_fwd_eager, *args)
+
+
+def rms_fwd_impl(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], bias: Optional[Tensor], eps: float,
+                 activation: int) -> Tensor:
     xc = x.contiguous()
     gc = None if gate is None else gate.to(xc.dtype).contiguous()
     wc = None if weight is None else weight.float().contiguous()
@@ -334,14 +419,16 @@ def rms_fwd(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], bias: O
     return y
 
 
+rms_fwd = torch.library.custom_op("sorernn::rms_norm_gated_fwd", mutates_args=())(rms_fwd_impl)
+
+
 @rms_fwd.register_fake
 def _rms_fwd_fake(x, gate, weight, bias, eps, activation):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("sorernn::rms_norm_gated_bwd", mutates_args=())
-def rms_bwd(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], bias: Optional[Tensor], dy: Tensor,
-            eps: float, activation: int) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+def rms_bwd_impl(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], bias: Optional[Tensor], dy: Tensor,
+                 eps: float, activation: int) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     xc = x.contiguous()
     gc = None if gate is None else gate.to(xc.dtype).contiguous()
     wc = None if weight is None else weight.float().contiguous()
@@ -362,6 +449,9 @@ def rms_bwd(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], bias: O
     return dx, dg, dw, db
 
 
+rms_bwd = torch.library.custom_op("sorernn::rms_norm_gated_bwd", mutates_args=())(rms_bwd_impl)
+
+
 @rms_bwd.register_fake
 def _rms_bwd_fake(x, gate, weight, bias, dy, eps, activation):
     d = x.shape[-1]
@@ -379,9 +469,15 @@ def _rms_setup(ctx, inputs, output):
 def _rms_backward(ctx, dy):
     x, gate, weight, bias = ctx.saved_tensors
     eps, activation = ctx.meta
-    dx, dg, dw, db = rms_bwd(x, gate, weight, bias, dy, eps, activation)
+    dx, dg, dw, db = _run_bwd(rms_bwd, rms_bwd_impl, x, gate, weight, bias, dy, eps, activation)
     return (dx, None if gate is None else dg.to(gate.dtype), None if weight is None else dw.to(weight.dtype),
             None if bias is None else db.to(bias.dtype), None, None)
 
 
 rms_fwd.register_autograd(_rms_backward, setup_context=_rms_setup)
+_rms_fwd_eager = _eager_function(rms_fwd_impl, _rms_setup, _rms_backward)
+
+
+def rms_fwd_call(*args):
+    """``rms_fwd`` as the Python entry points call it: directly when nothing traces or records."""
+    return _eager(rms_fwd, rms_fwd_impl, _rms_fwd_eager, *args)

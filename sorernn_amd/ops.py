@@ -134,11 +134,7 @@ def _delta_rule_args(name, q, k, v, g, beta, scale, initial_state, cu_seqlens, c
     return b, t, h, kd, hv, vd, n, flags, float(scale), A_log, dt_bias
 
 
-def _plain_eager(x: Tensor) -> bool:
-    """True for an ordinary tensor outside torch.compile, FX tracing and any active dispatch mode."""
-    return (type(x) is torch.Tensor and not torch.compiler.is_compiling()
-            and not torch.fx._symbolic_trace._is_fx_tracing_flag
-            and torch.utils._python_dispatch._get_current_dispatch_mode() is None)
+_plain_eager = _library.plain_eager  # an ordinary tensor outside compile, tracing, transforms and dispatch modes
 
 
 _recurrent_noted: set = set()
@@ -181,16 +177,15 @@ def _gdn_call(entry, name, q, k, v, g, beta, scale, initial_state, output_final_
     if entry == "gdn_chunk_fwd":
         # the torch.library op (sorernn::chunk_gated_delta_rule_fwd): traceable by torch.compile, with
         # the backward registered on it; with grad it also keeps the per-chunk states for the backward.
-        # Plain eager inference (no grad, no compile or fake tensors, no dispatch mode recording ops)
-        # calls the op's implementation directly: the dispatcher round trip costs more host time
-        # than the two kernel launches.
+        # Plain eager calls (no compile or fake tensors, no dispatch mode recording ops) run the op's
+        # implementation directly, under grad through an autograd function of it: the dispatcher round
+        # trip costs more host time than the kernel launches.
         eager = _plain_eager(q)
-        op = _library.chunk_fwd if (needs_grad or not eager) else _library.chunk_fwd_impl
         # the fp16 operand range guard (sorernn_amd/range_guard.py) reads its flag in eager calls only
         word = _range.before_call(q.device) if eager else None
-        o, final, _, _ = op(q, k, v, g, beta, initial_state, a_log_in if use_gate_in_kernel else None,
-                            dt_bias_in if use_gate_in_kernel else None, cu_seqlens, scale, flags, n,
-                            bool(output_final_state), needs_grad)
+        o, final, _, _ = _library.chunk_fwd_call(q, k, v, g, beta, initial_state, a_log_in if use_gate_in_kernel else None,
+                                                 dt_bias_in if use_gate_in_kernel else None, cu_seqlens, scale, flags, n,
+                                                 bool(output_final_state), needs_grad)
         if _range.call_overflowed(word, q.device):
             if _range.range_guard() == "raise" or needs_grad:
                 raise FloatingPointError(
@@ -522,7 +517,7 @@ def causal_conv1d(
     if initial_state is not None and tuple(initial_state.shape) != (n, c, w):
         raise ValueError(f"{name}: initial_state must be [N,C,W] = {(n, c, w)}")
     cu = cu_seqlens.contiguous() if cu_seqlens is not None else None
-    y, fin = _library.conv_fwd(x, weight, bias, initial_state, cu, act, flags, n, bool(output_final_state))
+    y, fin = _library.conv_fwd_call(x, weight, bias, initial_state, cu, act, flags, n, bool(output_final_state))
     return y, (fin if output_final_state else None)
 
 
@@ -611,7 +606,7 @@ def _l2norm_qk(q: Tensor, k: Tensor, eps: float = 1e-12) -> tuple[Tensor, Tensor
 def l2norm(x: Tensor, eps: float = 1e-12) -> Tensor:
     """``x / max(||x||_2, eps)`` over the last axis (``F.normalize`` semantics, fp32 math, one rounding)."""
     _check_cuda("l2norm", x)
-    return _library.l2norm_fwd(x, float(eps))
+    return _library.l2norm_fwd_call(x, float(eps))
 
 
 def rms_norm_gated(
@@ -644,4 +639,4 @@ def rms_norm_gated(
     d = x.shape[-1]
     if (weight is not None and weight.numel() != d) or (bias is not None and bias.numel() != d):
         raise ValueError(f"{name}: weight/bias must have {d} entries")
-    return _library.rms_fwd(x, g, weight, bias, float(eps), act)
+    return _library.rms_fwd_call(x, g, weight, bias, float(eps), act)

@@ -1,0 +1,111 @@
+"""CPU: which calls of the training operators go through the dispatcher and which run directly.
+
+The kernels are replaced by a recorder (the outputs' values are never looked at): plain eager calls must not
+enter the registered op, and every context that looks at operators must see it, as before the direct route.
+"""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from sorernn_amd import _lib, library
+
+
+class Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.ops = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.ops.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    entered = []
+    for name in ("chunk_fwd", "chunk_bwd", "conv_fwd", "conv_bwd", "l2norm_fwd", "l2norm_bwd", "rms_fwd", "rms_bwd"):
+        op = getattr(library, name)
+        monkeypatch.setattr(library, name, lambda *a, op=op, name=name: (entered.append(name), op(*a))[1])
+    return calls, entered
+
+
+def _x(*shape, grad=True):
+    return torch.randn(*shape).bfloat16().requires_grad_(grad)
+
+
+def _call(grad=True):
+    x, w = _x(1, 8, 16, grad=grad), torch.nn.Parameter(torch.randn(16, 4), requires_grad=grad)
+    return x, w, library.conv_fwd_call(x, w, None, None, None, 1, 0, 1, False)[0]
+
+
+def test_plain_calls_run_directly(launches):
+    calls, entered = launches
+    _call(grad=False)
+    x, w, y = _call()
+    torch.autograd.grad(y, [x, w], torch.ones_like(y))
+    n = library.l2norm_fwd_call(x.view(8, 16), 1e-12)
+    z = library.rms_fwd_call(n, n.detach(), torch.nn.Parameter(torch.ones(16)), None, 1e-6, 1)
+    z.sum().backward()
+    q, v, g = _x(1, 8, 1, 64), _x(1, 8, 1, 64), torch.zeros(1, 8, 1, requires_grad=True)
+    o, fin, states, ws = library.chunk_fwd_call(q, q, v, g, g, None, None, None, None, 0.125, 0, 1, True, True)
+    assert o.requires_grad and fin.requires_grad and not states.requires_grad and not ws.requires_grad
+    torch.autograd.grad([o, fin], [q, v, g], [torch.ones_like(o), torch.ones_like(fin)])
+    assert not entered
+    assert calls == ["gdn_causal_conv1d_fwd", "gdn_causal_conv1d_fwd", "gdn_causal_conv1d_bwd", "gdn_l2norm_fwd",
+                     "gdn_rms_norm_gated_fwd", "gdn_rms_norm_gated_bwd", "gdn_l2norm_bwd", "gdn_chunk_fwd_train",
+                     "gdn_chunk_bwd"]
+
+
+def test_dispatch_modes_see_the_op(launches):
+    with Seen() as seen:
+        x, w, y = _call()
+        torch.autograd.grad(y, [x, w], torch.ones_like(y))
+    assert any("causal_conv1d_fwd" in s for s in seen.ops) and any("causal_conv1d_bwd" in s for s in seen.ops)
+
+
+def test_transforms_and_subclasses_take_the_op(launches):
+    calls, entered = launches
+
+    class Sub(torch.Tensor):
+        pass
+
+    x = torch.randn(8, 16).bfloat16()
+    library.l2norm_fwd_call(x.as_subclass(Sub), 1e-12)
+    assert entered.pop() == "l2norm_fwd" and not entered
+    with torch.autograd.forward_ad.dual_level():
+        library.l2norm_fwd_call(x, 1e-12)
+    assert entered.pop() == "l2norm_fwd" and not entered
+    calls.clear()
+    y = torch.vmap(lambda t: library.l2norm_fwd_call(t, 1e-12))(x.view(2, 4, 16))  # torch's loop over the op
+    assert entered.pop() == "l2norm_fwd" and not entered and calls == ["gdn_l2norm_fwd"] * 2 and y.shape == (2, 4, 16)
+    y = torch.fx.experimental.proxy_tensor.make_fx(lambda t: library.l2norm_fwd_call(t, 1e-12))(x)
+    assert any("l2norm_fwd" in str(n.target) for n in y.graph.nodes)
+
+
+def test_saved_tensor_hooks_and_second_derivatives(launches):
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t)[1], lambda t: t):
+        x, w, y = _call()
+    assert torch.Size([1, 8, 16]) in packed and torch.Size([16, 4]) in packed
+    (dx,) = torch.autograd.grad(y, x, torch.ones_like(y), create_graph=True)
+    with pytest.raises(RuntimeError):
+        dx.sum().backward()
+
+
+def test_compiled_call_holds_the_op(launches):
+    graphs = []
+
+    def keep(gm, _):
+        graphs.append(gm)
+        return gm.forward
+
+    torch._dynamo.reset()
+    fn = torch.compile(lambda t, w: library.conv_fwd_call(t, w, None, None, None, 1, 0, 1, False)[0], backend=keep, fullgraph=True)
+    try:
+        fn(torch.randn(1, 8, 16).bfloat16(), torch.randn(16, 4))
+    finally:
+        torch._dynamo.reset()
+    assert any("causal_conv1d_fwd" in str(n.target) for n in graphs[0].graph.nodes)
