@@ -144,12 +144,12 @@ __device__ __forceinline__ void fetch_qk(QKRows<KD, NT>& r, const bf16* src, int
   for (int u = 0; u < R::N; ++u) r.x[u] = buf_load16(rs, (uint32_t)(row + u * R::RPP) * rb + ch * 16);
 }
 template <int KD, int NT>
-__device__ __forceinline__ void put_qk(const QKRows<KD, NT>& r, bf16* dst, int pitch, bool l2, int tid) {
+__device__ __forceinline__ void put_qk(QKRows<KD, NT>& r, bf16* dst, int pitch, bool l2, int tid) {
   using R = QKRows<KD, NT>;
   const int row = tid / R::KCH, ch = tid % R::KCH;
+  if (l2) l2norm_row_chunks<R::KCH>(r.x);
 #pragma unroll
-  for (int u = 0; u < R::N; ++u)
-    *reinterpret_cast<bf16x8*>(dst + (row + u * R::RPP) * pitch + ch * 8) = l2 ? l2norm_row_chunk<R::KCH>(r.x[u]) : r.x[u];
+  for (int u = 0; u < R::N; ++u) *reinterpret_cast<bf16x8*>(dst + (row + u * R::RPP) * pitch + ch * 8) = r.x[u];
 }
 // A [64][W] slice (16-byte pieces) of a [tokens][heads][*] tensor with row stride rb bytes.
 template <int W, int NT>
@@ -311,11 +311,14 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_bwd_prep_kernel(ChunkBw
 }
 
 // ================================================================== 2. reverse state recurrence
-// One workgroup of 4 waves per (sequence, value head, 32 value columns). Waves 0 and 1 each hold 16
+// One workgroup per (sequence, value head, 32 value columns). Waves 0 and 1 each hold 16
 // columns of dS [K x 16] in fp32 MFMA accumulators (tile a: keys 16a + 4g + r, column i) for the
-// whole sequence; waves 2 and 3 stage the next chunk's tiles into the other LDS slot meanwhile.
+// whole sequence; waves 2, 3, 6 and 7 stage the next chunk's tiles into the other LDS slot meanwhile (the SIMDs
+// without a state wave; waves 4 and 5, which would share the state waves' SIMDs, only keep the barriers).
+// Config 1 with the q/k norm: 206 us with two loader waves, each lane normalising its 16 row pieces one by one,
+// 152 us with four and the pieces side by side.
 template <int KD, int VD>
-__global__ __launch_bounds__(256, 1) void gated_delta_chunk_bwd_state_kernel(ChunkBwdParams p) {
+__global__ __launch_bounds__(512, 1) void gated_delta_chunk_bwd_state_kernel(ChunkBwdParams p) {
   constexpr int KPB = row_pitch<KD>(), KS = KD / 32, KT = KD / 16, NVB = VD / 32;
   constexpr int OP = 40;  // bf16 pitch of the dO slice
   __shared__ __align__(16) bf16 Kb[2][kC * KPB], Qb[2][kC * KPB], Tm[2][kC * kCPb], dOs[2][kC * OP];
@@ -351,13 +354,13 @@ __global__ __launch_bounds__(256, 1) void gated_delta_chunk_bwd_state_kernel(Chu
   const int nc = (int)((eos - bos + kC - 1) / kC);
   const bool l2 = p.flags & GDN_FLAG_QK_L2NORM;
 
-  // Loader waves (2, 3; tl = 0..127): a chunk's tiles are fetched into registers a step before they
+  // Loader waves (2, 3, 6, 7; tl = 0..255): a chunk's tiles are fetched into registers a step before they
   // are written to LDS, so each step hides a step of load latency.
   struct ChunkRegs {
-    QKRows<KD, 128> xk, xq;
-    Slice<kC, 128> xt;
-    Slice<32, 128> xo;
-    u32x4 xg[2];  // the G1 slice: 32 columns x 64 tokens, 4 KB contiguous in the chunk-blocked G1
+    QKRows<KD, 256> xk, xq;
+    Slice<kC, 256> xt;
+    Slice<32, 256> xo;
+    u32x4 xg;  // the G1 slice: 32 columns x 64 tokens, 4 KB contiguous in the chunk-blocked G1
     uint32_t graw, braw;
     int len;
   };
@@ -370,21 +373,16 @@ __global__ __launch_bounds__(256, 1) void gated_delta_chunk_bwd_state_kernel(Chu
     fetch_slice(r.xo, static_cast<const bf16*>(p.dout) + (c0 * p.HV + hv) * VD + vb * 32, (uint32_t)(p.HV * VD * 2),
                 r.len, tl);
     const bf16* g1src = p.g1 + (((cgb + c) * p.HV + hv) * VD + vb * 32) * kC;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) r.xg[u] = *reinterpret_cast<const u32x4*>(g1src + (u * 128 + tl) * 8);
+    r.xg = *reinterpret_cast<const u32x4*>(g1src + tl * 8);
     r.graw = r.braw = 0;
     if (w == 2) fetch_gates_bwd(r.graw, r.braw, p, c0, hv, r.len, lane);
   };
-  auto put_chunk = [&](const ChunkRegs& r, int slot, int tl) {
+  auto put_chunk = [&](ChunkRegs& r, int slot, int tl) {
     put_qk(r.xk, Kb[slot], KPB, l2, tl);
     put_qk(r.xq, Qb[slot], KPB, l2, tl);
     put_slice(r.xt, Tm[slot], kCPb, tl);
     put_slice(r.xo, dOs[slot], OP, tl);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int e = u * 128 + tl;  // column e / 8, tokens 8 (e % 8) .. + 7
-      *reinterpret_cast<u32x4*>(G1s[slot] + (e >> 3) * kCPb + (e & 7) * 8) = r.xg[u];
-    }
+    *reinterpret_cast<u32x4*>(G1s[slot] + (tl >> 3) * kCPb + (tl & 7) * 8) = r.xg;  // column tl / 8, tokens 8 (tl % 8) .. + 7
     if (w == 2) put_gates_bwd(gv[slot], r.graw, r.braw, p, hv, r.len, lane);
   };
 
@@ -518,8 +516,8 @@ __global__ __launch_bounds__(256, 1) void gated_delta_chunk_bwd_state_kernel(Chu
 #pragma unroll
         for (int r = 0; r < 4; ++r) p.dh0[((n * p.HV + hv) * KD + 16 * a + 4 * g4 + r) * VD + col] = dS[a][r];
     }
-  } else {
-    const int tl = t - 128;
+  } else if (w & 2) {
+    const int tl = ((w >> 2) * 2 + (w & 1)) * kWave + lane;
     ChunkRegs nx;  // the next chunk's tiles, in flight across a step
     if (nc > 0) {
       fetch_chunk(nx, nc - 1, tl);
@@ -535,6 +533,8 @@ __global__ __launch_bounds__(256, 1) void gated_delta_chunk_bwd_state_kernel(Chu
       }
       __syncthreads();
     }
+  } else {
+    for (int i = 0; i <= nc; ++i) __syncthreads();
   }
 }
 
@@ -1130,7 +1130,7 @@ extern "C" int gdn_chunk_bwd(const void* q, const void* k, const void* v, const 
   GDN_BWD_DISPATCH(gated_delta_chunk_bwd_prep_kernel, dim3((unsigned)chunks, (unsigned)HV), dim3(256));
   int rc = gdn_internal_check_launch("gated_delta_chunk_bwd_prep_kernel");
   if (rc != GDN_OK) return rc;
-  GDN_BWD_DISPATCH(gated_delta_chunk_bwd_state_kernel, dim3((unsigned)(N * HV * (V / 32))), dim3(256));
+  GDN_BWD_DISPATCH(gated_delta_chunk_bwd_state_kernel, dim3((unsigned)(N * HV * (V / 32))), dim3(512));
   rc = gdn_internal_check_launch("gated_delta_chunk_bwd_state_kernel");
   if (rc != GDN_OK) return rc;
   GDN_BWD_DISPATCH(gated_delta_chunk_bwd_grad_kernel, dim3((unsigned)chunks, (unsigned)H), dim3(256));
