@@ -23,6 +23,7 @@ struct ConvParams {
   int cu_i32;
   int64_t T, C, N;
   int dx, act;
+  int tt;  // tokens per thread of the vector kernel
 };
 
 constexpr int kConvTokens = 64;
@@ -95,27 +96,38 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_kernel(ConvParams p) {
   }
 }
 
-// Vector path for 16-bit activations with C % 8 == 0: each thread owns 8 consecutive channels
-// (16-byte loads and stores of a token row; a wave covers 512 channels, 1 KB per token) and walks
-// kConvV8Tokens tokens, issuing the loads of 8 token rows before it uses the first. Same
-// semantics and document handling as gated_delta_conv1d_kernel.
-constexpr int kConvV8Tokens = 32;
+// Tokens a thread of the two vector kernels below walks: the longest segment (each re-reads the 3 rows before it)
+// that still gives 3,072 waves, 3 per SIMD: fewer leave loads unhidden, and a short call is one thread's serial walk.
+// bf16, us at 16 / 32 / 64 tokens: conv of 16,384 x 2,048 29.3 / 30.7 / 34.0, of 4,096 x 2,048 13.0 / 17.6 / 29.1
+// (12.5 at 8), of 1,000 x 2,048 9.4 / 15.1 / 26.1 (6.3 at 8); the q/k/v prologue of 2 x 8,192 tokens x 6,144
+// channels 100.9 / 106.3 / 95.5, of 2,048 tokens 19.2 / 21.0 / 34.8 (18.4 at 8).
+static int conv_tokens(int64_t B, int64_t T, int64_t waves_x) {
+  int tt = 64;
+  while (tt > 8 && B * ((T + tt - 1) / tt) * waves_x < 3072) tt /= 2;
+  return tt;
+}
 
+// Vector path for C % V == 0: each thread owns V consecutive channels, 16 bytes of a token row (V = 8 of a 16-bit
+// type, 4 of fp32; a wave covers 1 KB per token), and walks p.tt tokens, issuing the loads of 8 token
+// rows before it uses the first. Same semantics and document handling as gated_delta_conv1d_kernel. HBM-bound:
+// 134 MB in 29 us at 16,384 x 2,048 in bf16 (4.6 TB/s).
 template <int W, typename E>
-__global__ __launch_bounds__(256) void gated_delta_conv1d_v8_kernel(ConvParams p) {
-  typedef E V8 __attribute__((ext_vector_type(8)));
-  const int64_t c0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+__global__ __launch_bounds__(256) void gated_delta_conv1d_vec_kernel(ConvParams p) {
+  constexpr int V = 16 / sizeof(E);
+  constexpr bool kFast = sizeof(E) == 2;  // outputs rounded to 16 bits: SiLU from v_exp_f32 / v_rcp_f32
+  typedef E V8 __attribute__((ext_vector_type(V)));
+  const int64_t c0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (c0 >= p.C) return;
   const int64_t bb = blockIdx.z;
-  const int64_t t0 = (int64_t)blockIdx.y * kConvV8Tokens;
+  const int64_t t0 = (int64_t)blockIdx.y * p.tt;
   if (t0 >= p.T) return;
-  const int64_t t1 = t0 + kConvV8Tokens < p.T ? t0 + kConvV8Tokens : p.T;
+  const int64_t t1 = t0 + p.tt < p.T ? t0 + p.tt : p.T;
   const E* __restrict__ xs = static_cast<const E*>(p.x) + bb * p.T * p.C + c0;
   E* __restrict__ ys = static_cast<E*>(p.y) + bb * p.T * p.C + c0;
   const E* init = static_cast<const E*>(p.init);
-  float w[8][W], bias[8];
+  float w[V][W], bias[V];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
+  for (int e = 0; e < V; ++e) {
 #pragma unroll
     for (int i = 0; i < W; ++i) w[e][i] = p.w[(c0 + e) * W + i];
     bias[e] = p.bias ? p.bias[c0 + e] : 0.f;
@@ -133,17 +145,17 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_v8_kernel(ConvParams p
     de = load_index(p.cu, p.cu_i32, d + 1);
   }
   // win[i][e]: input at position t - (W-1) + i of channel c0 + e for the next token t
-  float win[W > 1 ? W - 1 : 1][8];
+  float win[W > 1 ? W - 1 : 1][V];
 #pragma unroll
   for (int i = 0; i < W - 1; ++i) {
     const int64_t pos = t0 - (W - 1) + i;
     if (pos >= ds) {
       const V8 v = *reinterpret_cast<const V8*>(xs + pos * p.C);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) win[i][e] = (float)v[e];
+      for (int e = 0; e < V; ++e) win[i][e] = (float)v[e];
     } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) win[i][e] = init ? (float)init[(d * p.C + c0 + e) * W + (W - (ds - pos))] : 0.f;
+      for (int e = 0; e < V; ++e) win[i][e] = init ? (float)init[(d * p.C + c0 + e) * W + (W - (ds - pos))] : 0.f;
     }
   }
   for (int64_t tg = t0; tg < t1; tg += 8) {
@@ -164,17 +176,17 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_v8_kernel(ConvParams p
 #pragma unroll
         for (int i = 0; i < W - 1; ++i)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) win[i][e] = init ? (float)init[(d * p.C + c0 + e) * W + i + 1] : 0.f;
+          for (int e = 0; e < V; ++e) win[i][e] = init ? (float)init[(d * p.C + c0 + e) * W + i + 1] : 0.f;
       }
       V8 yv;
-      float xt[8], dropped[8];
+      float xt[V], dropped[V];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < V; ++e) {
         xt[e] = (float)xv[g][e];
         float acc = bias[e] + w[e][W - 1] * xt[e];
 #pragma unroll
         for (int i = 0; i < W - 1; ++i) acc += w[e][i] * win[i][e];
-        if (p.act == GDN_ACT_SILU) acc = silu_fast(acc);
+        if (p.act == GDN_ACT_SILU) acc = kFast ? silu_fast(acc) : silu_f32(acc);
         yv[e] = (E)acc;
         dropped[e] = W > 1 ? win[0][e] : xt[e];
 #pragma unroll
@@ -185,7 +197,7 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_v8_kernel(ConvParams p
       if (p.fin && t == de - 1) {  // last token of document d: the cache is its last W inputs
         E* fin = static_cast<E*>(p.fin);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < V; ++e) {
           const int64_t fb = (d * p.C + c0 + e) * W;
           if (W > 1) {
             fin[fb] = (E)dropped[e];
@@ -206,7 +218,7 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_v8_kernel(ConvParams p
 // stores it, then, with l2, each q and k head of D channels L2-normalised (x / max(|x|, 1e-12) as
 // v_rsq_f32 of max(|x|^2, 1e-24), the chunk kernels' in-kernel formula; fp32 math, rounded again)
 // -> contiguous q, k [B, T, Cqk] and v [B, T, Cv].
-// Thread = 8 channels as in gated_delta_conv1d_v8_kernel; a head of D channels is D/8 consecutive
+// Thread = 8 channels as in gated_delta_conv1d_vec_kernel; a head of D channels is D/8 consecutive
 // lanes, so its sum of squares is a DPP group sum. No conv caches (the layer's forward uses none).
 // The activation and the varlen document walk are template parameters, so the unrolled row loop has
 // no branches on them (with the reciprocal square root: 110 -> 104 us at config 4's shape).
@@ -220,6 +232,7 @@ struct QkvConvParams {
   int cu_i32;
   int64_t T, Cqk, Cv, N;
   int act, l2;
+  int tt;  // tokens per thread
 };
 
 template <typename E, int D, int ACT, bool VARLEN>
@@ -233,9 +246,9 @@ __global__ __launch_bounds__(256) void gated_delta_qkv_conv1d_kernel(QkvConvPara
   const bool ch_ok = c0 < ctot;
   const int64_t cc = ch_ok ? c0 : ctot - 8;
   const int64_t bb = blockIdx.z;
-  const int64_t t0 = (int64_t)blockIdx.y * kConvV8Tokens;
+  const int64_t t0 = (int64_t)blockIdx.y * p.tt;
   if (t0 >= p.T) return;
-  const int64_t t1 = t0 + kConvV8Tokens < p.T ? t0 + kConvV8Tokens : p.T;
+  const int64_t t1 = t0 + p.tt < p.T ? t0 + p.tt : p.T;
   const E* __restrict__ xs = static_cast<const E*>(p.x) + bb * p.T * p.x_stride + cc;
   // output and its channel offset: q | k | v
   E* dst;
@@ -679,15 +692,17 @@ extern "C" int gdn_causal_conv1d_fwd(const void* x, const float* weight, const f
     return GDN_ERR_UNSUPPORTED;
   }
   ConvParams p{x, weight, bias, y, initial_state, final_state, cu_seqlens, (flags & GDN_FLAG_CU_INT32) ? 1 : 0,
-               T, C, N, x_dtype, activation};
+               T, C, N, x_dtype, activation, 0};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t tb8 = (T + kConvV8Tokens - 1) / kConvV8Tokens;
+  const int V = x_dtype == GDN_DTYPE_F32 ? 4 : 8;  // channels per thread of the vector kernel
   const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
-  if (aligned && C % 8 == 0 && W == 4 && tb8 <= 65535 && (x_dtype == GDN_DTYPE_BF16 || x_dtype == GDN_DTYPE_F16)) {
-    const dim3 g8((unsigned)((C / 8 + 255) / 256), (unsigned)tb8, (unsigned)B), b8(256);
-    if (x_dtype == GDN_DTYPE_BF16) hipLaunchKernelGGL((gated_delta_conv1d_v8_kernel<4, bf16>), g8, b8, 0, s, p);
-    else hipLaunchKernelGGL((gated_delta_conv1d_v8_kernel<4, f16>), g8, b8, 0, s, p);
-    return gdn_internal_check_launch("gated_delta_conv1d_v8_kernel");
+  if (aligned && C % V == 0 && W == 4) {
+    p.tt = conv_tokens(B, T, (C / V + 63) / 64);
+    const dim3 gv((unsigned)((C / V + 255) / 256), (unsigned)((T + p.tt - 1) / p.tt), (unsigned)B), bv(256);
+    if (x_dtype == GDN_DTYPE_BF16) hipLaunchKernelGGL((gated_delta_conv1d_vec_kernel<4, bf16>), gv, bv, 0, s, p);
+    else if (x_dtype == GDN_DTYPE_F16) hipLaunchKernelGGL((gated_delta_conv1d_vec_kernel<4, f16>), gv, bv, 0, s, p);
+    else hipLaunchKernelGGL((gated_delta_conv1d_vec_kernel<4, float>), gv, bv, 0, s, p);
+    return gdn_internal_check_launch("gated_delta_conv1d_vec_kernel");
   }
   dim3 grid((unsigned)((C + 255) / 256), (unsigned)tb, (unsigned)B), block(256);
   switch (W) {
@@ -826,15 +841,15 @@ extern "C" int gdn_qkv_conv_fwd(const void* x, int64_t x_row_stride, const float
     return GDN_ERR_INVALID;
   }
   if (T == 0) return GDN_OK;
-  const int64_t tb = (T + kConvV8Tokens - 1) / kConvV8Tokens;
-  if (tb > 65535 || B > 65535) {
+  if (T > (int64_t)65535 * 32 || B > 65535) {
     gdn_internal_set_error("gdn_qkv_conv_fwd: T=%lld B=%lld exceed the grid limits", (long long)T, (long long)B);
     return GDN_ERR_UNSUPPORTED;
   }
   QkvConvParams p{x, x_row_stride, weight, bias, q, k, v, cu_seqlens, (flags & GDN_FLAG_CU_INT32) ? 1 : 0, T, Cqk, Cv,
-                  N, activation, (flags & GDN_FLAG_QK_L2NORM) ? 1 : 0};
+                  N, activation, (flags & GDN_FLAG_QK_L2NORM) ? 1 : 0, 0};
   const int64_t threads = (2 * Cqk + Cv) / 8;
-  const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)tb, (unsigned)B), block(256);
+  p.tt = conv_tokens(B, T, (threads + 63) / 64);
+  const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)((T + p.tt - 1) / p.tt), (unsigned)B), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
   // dtype, head dim, activation and varlen as template arguments
   auto go = [&](auto e_tag, auto d_c, auto a_c, auto v_c) {
