@@ -21,6 +21,10 @@ import torch
 from torch import Tensor
 from torch.autograd import forward_ad
 from torch.autograd.function import once_differentiable
+from torch._C import _functorch
+from torch.fx import _symbolic_trace
+from torch.nn import Parameter
+from torch.utils import _python_dispatch
 
 from sorernn_amd import _lib
 
@@ -32,11 +36,11 @@ def plain_eager(*tensors) -> bool:
     compile or FX tracing, no dispatch mode, no functorch transform (vmap, grad, jvp), no forward-mode level."""
     if torch.compiler.is_compiling():
         return False
-    return (all(t is None or type(t) is Tensor or type(t) is torch.nn.Parameter for t in tensors)
-            and not torch.fx._symbolic_trace._is_fx_tracing_flag
-            and torch.utils._python_dispatch._get_current_dispatch_mode() is None
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and forward_ad._current_level < 0)
+    for t in tensors:
+        if type(t) is not Tensor and type(t) is not Parameter and t is not None:
+            return False
+    return (not _symbolic_trace._is_fx_tracing_flag and _python_dispatch._get_current_dispatch_mode() is None
+            and _functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0)
 
 
 def _eager_function(impl, setup, backward):

@@ -183,9 +183,10 @@ def _gdn_call(entry, name, q, k, v, g, beta, scale, initial_state, output_final_
         eager = _plain_eager(q)
         # the fp16 operand range guard (sorernn_amd/range_guard.py) reads its flag in eager calls only
         word = _range.before_call(q.device) if eager else None
-        o, final, _, _ = _library.chunk_fwd_call(q, k, v, g, beta, initial_state, a_log_in if use_gate_in_kernel else None,
-                                                 dt_bias_in if use_gate_in_kernel else None, cu_seqlens, scale, flags, n,
-                                                 bool(output_final_state), needs_grad)
+        op = _library.chunk_fwd_call if needs_grad else _library.chunk_fwd_impl if eager else _library.chunk_fwd
+        o, final, _, _ = op(q, k, v, g, beta, initial_state, a_log_in if use_gate_in_kernel else None,
+                            dt_bias_in if use_gate_in_kernel else None, cu_seqlens, scale, flags, n,
+                            bool(output_final_state), needs_grad)
         if _range.call_overflowed(word, q.device):
             if _range.range_guard() == "raise" or needs_grad:
                 raise FloatingPointError(
