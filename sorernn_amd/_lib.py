@@ -97,6 +97,10 @@ def load() -> ctypes.CDLL:
     ver = lib.gdn_abi_version()
     if ver != ABI_VERSION:
         raise RuntimeError(f"libgdn.so ABI version {ver} != expected {ABI_VERSION}; rebuild it")
+    # Reads the library's thread-local error text once. glibc refreshes a thread's table of thread-local blocks only
+    # when it reaches the newest library's; until then every torch call from it takes the slow lookup (x.data_ptr()
+    # 0.10 us instead of 0.08; a decode step's call 10.8 us instead of 9.1).
+    lib.gdn_last_error()
     _lib = lib
     return lib
 
