@@ -20,7 +20,6 @@ from typing import Optional
 import torch
 from torch import Tensor
 from torch.autograd import forward_ad
-from torch.autograd.function import once_differentiable
 from torch._C import _functorch
 from torch.fx import _symbolic_trace
 from torch.nn import Parameter
@@ -47,7 +46,9 @@ def _eager_function(impl, setup, backward):
     """The autograd function of an op for plain eager calls: the op's implementation, context and formula without
     the dispatcher and the custom-op wrappers, which cost the host more per call than the kernels run (a conv
     forward and backward of 4,096 x 2,048 tokens takes 40 us on the GPU, its host work took 160 us and takes 100). Saved tensors go through
-    ``save_for_backward`` as there (hooks see them); a second derivative raises, as there."""
+    ``save_for_backward`` as there (hooks see them). The backward is not marked ``once_differentiable``: that marks the
+    gradients only where an incoming one requires grad, and under ``create_graph`` with a constant incoming gradient
+    (``y.sum()``) they would look like constants of the inputs. ``_run_bwd`` enters the op there instead."""
 
     class EagerOp(torch.autograd.Function):
         @staticmethod
@@ -59,7 +60,6 @@ def _eager_function(impl, setup, backward):
             return out
 
         @staticmethod
-        @once_differentiable
         def backward(ctx, *grads):
             return backward(ctx, *grads)
 

@@ -91,8 +91,38 @@ def test_saved_tensor_hooks_and_second_derivatives(launches):
         x, w, y = _call()
     assert torch.Size([1, 8, 16]) in packed and torch.Size([16, 4]) in packed
     (dx,) = torch.autograd.grad(y, x, torch.ones_like(y), create_graph=True)
-    with pytest.raises(RuntimeError):
+    with pytest.raises(RuntimeError, match="autograd formula"):
         dx.sum().backward()
+
+
+def _chunk(q, v, g):
+    return library.chunk_fwd_call(q, q, v, g, g, None, None, None, None, 0.125, 0, 1, False, True)[0]
+
+
+def _forwards():
+    """(name of the backward op, forward of one tensor that requires grad) of every differentiable operator."""
+    w, n, g = torch.randn(16, 4), torch.ones(16), torch.zeros(1, 8, 1)
+    return [
+        ("conv_bwd", lambda x: library.conv_fwd_call(x.view(1, 8, 16), w, None, None, None, 1, 0, 1, False)[0]),
+        ("l2norm_bwd", lambda x: library.l2norm_fwd_call(x, 1e-12)),
+        ("rms_bwd", lambda x: library.rms_fwd_call(x, None, n, None, 1e-6, 0)),
+        ("chunk_bwd", lambda x: _chunk(x.view(1, 2, 1, 64), x.view(1, 2, 1, 64), g[:, :2])),
+    ]
+
+
+@pytest.mark.parametrize("grad_needs_grad", [False, True])
+@pytest.mark.parametrize("which", range(4))
+def test_second_derivatives_raise(launches, which, grad_needs_grad):
+    """A gradient taken with ``create_graph`` depends on the inputs whether or not the incoming one requires grad: a loss
+    that holds it next to a differentiable term raises, as no second derivative exists, and is not merely cut short."""
+    name, fn = _forwards()[which]
+    x, other = _x(8, 16), torch.ones(1, requires_grad=True)
+    y = fn(x)
+    launches[1].clear()
+    (dx,) = torch.autograd.grad(y, x, torch.ones_like(y).requires_grad_(grad_needs_grad), create_graph=True)
+    assert launches[1] == [name] and dx.requires_grad
+    with pytest.raises(RuntimeError, match="autograd formula"):
+        (dx.float().square().sum() + other).backward()
 
 
 def test_compiled_call_holds_the_op(launches):
