@@ -20,7 +20,7 @@ from typing import Optional
 import torch
 from torch import Tensor
 from torch.autograd import forward_ad
-from torch._C import _functorch
+from torch._C import _functorch, _get_tracing_state
 from torch.fx import _symbolic_trace
 from torch.nn import Parameter
 from torch.utils import _python_dispatch
@@ -32,14 +32,16 @@ C = 64  # chunk length
 
 def plain_eager(*tensors) -> bool:
     """True when nothing but the autograd engine looks at these tensors' operators: ordinary tensors, no
-    compile or FX tracing, no dispatch mode, no functorch transform (vmap, grad, jvp), no forward-mode level."""
+    compile, FX or ``torch.jit`` tracing, no dispatch mode, no functorch transform (vmap, grad, jvp), no forward-mode
+    level."""
     if torch.compiler.is_compiling():
         return False
     for t in tensors:
         if type(t) is not Tensor and type(t) is not Parameter and t is not None:
             return False
     return (not _symbolic_trace._is_fx_tracing_flag and _python_dispatch._get_current_dispatch_mode() is None
-            and _functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0)
+            and _functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
+            and _get_tracing_state() is None)
 
 
 def _eager_function(impl, setup, backward):

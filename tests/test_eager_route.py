@@ -125,6 +125,14 @@ def test_second_derivatives_raise(launches, which, grad_needs_grad):
         (dx.float().square().sum() + other).backward()
 
 
+@pytest.mark.parametrize("which", range(4))
+def test_jit_traces_hold_the_op(launches, which):
+    """A trace that missed the operator would hold its outputs' allocations alone and return uninitialised memory."""
+    _, fn = _forwards()[which]
+    graph = torch.jit.trace(fn, _x(8, 16, grad=False), check_trace=False).graph
+    assert any(n.kind().startswith("sorernn::") for n in graph.nodes()), graph
+
+
 def test_compiled_call_holds_the_op(launches):
     graphs = []
 
