@@ -33,11 +33,11 @@ C = 64  # chunk length
 def plain_eager(*tensors) -> bool:
     """True when nothing but the autograd engine looks at these tensors' operators: ordinary tensors, no
     compile, FX or ``torch.jit`` tracing, no dispatch mode, no functorch transform (vmap, grad, jvp), no forward-mode
-    level."""
+    level, no batched tensor of the vmap that ``is_grads_batched`` runs under (its type is ``Tensor`` as well)."""
     if torch.compiler.is_compiling():
         return False
     for t in tensors:
-        if type(t) is not Tensor and type(t) is not Parameter and t is not None:
+        if t is not None and ((type(t) is not Tensor and type(t) is not Parameter) or _functorch.is_legacy_batchedtensor(t)):
             return False
     return (not _symbolic_trace._is_fx_tracing_flag and _python_dispatch._get_current_dispatch_mode() is None
             and _functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0

@@ -126,6 +126,21 @@ def test_second_derivatives_raise(launches, which, grad_needs_grad):
 
 
 @pytest.mark.parametrize("which", range(4))
+def test_batched_gradients_loop_over_the_op(launches, which):
+    """``is_grads_batched`` and vectorised Jacobians: one launch of the backward per gradient."""
+    calls, entered = launches
+    name, fn = _forwards()[which]
+    x = _x(8, 16)
+    y = fn(x)
+    calls.clear(), entered.clear()
+    (dx,) = torch.autograd.grad(y, x, torch.ones(3, *y.shape, dtype=y.dtype), is_grads_batched=True)
+    assert dx.shape == (3, 8, 16) and entered == [name] and len(calls) == 3
+    calls.clear()
+    jac = torch.autograd.functional.jacobian(lambda t: fn(t).float().sum().view(1), x.detach(), vectorize=True)
+    assert jac.shape == (1, 8, 16) and len(calls) == 2
+
+
+@pytest.mark.parametrize("which", range(4))
 def test_jit_traces_hold_the_op(launches, which):
     """A trace that missed the operator would hold its outputs' allocations alone and return uninitialised memory."""
     _, fn = _forwards()[which]
