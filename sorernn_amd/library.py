@@ -19,8 +19,8 @@ from typing import Optional
 
 import torch
 from torch import Tensor
-from torch.autograd import forward_ad
-from torch._C import _functorch, _get_tracing_state
+from torch.autograd import forward_ad, profiler
+from torch._C import _functorch, _get_tracing_state, _is_torch_function_mode_enabled
 from torch.fx import _symbolic_trace
 from torch.nn import Parameter
 from torch.utils import _python_dispatch
@@ -33,7 +33,8 @@ C = 64  # chunk length
 def plain_eager(*tensors) -> bool:
     """True when nothing but the autograd engine looks at these tensors' operators: ordinary tensors, no
     compile, FX or ``torch.jit`` tracing, no dispatch mode, no functorch transform (vmap, grad, jvp), no forward-mode
-    level, no batched tensor of the vmap that ``is_grads_batched`` runs under (its type is ``Tensor`` as well)."""
+    level, no batched tensor of the vmap that ``is_grads_batched`` runs under (its type is ``Tensor`` as well), no
+    torch-function mode, and no running profiler (it records the registered ops)."""
     if torch.compiler.is_compiling():
         return False
     for t in tensors:
@@ -41,7 +42,8 @@ def plain_eager(*tensors) -> bool:
             return False
     return (not _symbolic_trace._is_fx_tracing_flag and _python_dispatch._get_current_dispatch_mode() is None
             and _functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
-            and _get_tracing_state() is None)
+            and _get_tracing_state() is None and not _is_torch_function_mode_enabled()
+            and not profiler._is_profiler_enabled)
 
 
 def _eager_function(impl, setup, backward):

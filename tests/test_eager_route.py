@@ -5,6 +5,7 @@ enter the registered op, and every context that looks at operators must see it, 
 """
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from sorernn_amd import _lib, library
@@ -123,6 +124,32 @@ def test_second_derivatives_raise(launches, which, grad_needs_grad):
     assert launches[1] == [name] and dx.requires_grad
     with pytest.raises(RuntimeError, match="autograd formula"):
         (dx.float().square().sum() + other).backward()
+
+
+class SeenFunctions(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.ops = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.ops.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("which", range(4))
+def test_function_modes_and_the_profiler_see_the_op(launches, which):
+    name, fn = _forwards()[which]
+    x = _x(8, 16)
+    with SeenFunctions() as seen:
+        y = fn(x)
+    assert any(s.startswith("sorernn.") for s in seen.ops), seen.ops
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        fn(x).sum().backward()
+    ops = {e.name for e in prof.events() if e.name.startswith("sorernn::")}
+    assert len(ops) == 2, ops
+    launches[1].clear()
+    y.sum().backward()
+    assert not launches[1]
 
 
 @pytest.mark.parametrize("which", range(4))
