@@ -30,18 +30,27 @@ from sorernn_amd import _lib
 C = 64  # chunk length
 
 
-def plain_eager(*tensors) -> bool:
-    """True when nothing but the autograd engine looks at these tensors' operators: ordinary tensors, no
-    compile, FX or ``torch.jit`` tracing, no dispatch mode, no functorch transform (vmap, grad, jvp), no forward-mode
-    level, no batched tensor of the vmap that ``is_grads_batched`` runs under (its type is ``Tensor`` as well), no
-    torch-function mode, and no running profiler (it records the registered ops)."""
+def ordinary(*tensors) -> bool:
+    """True for ordinary tensors outside compile, FX tracing and dispatch modes: their values exist when a call returns."""
     if torch.compiler.is_compiling():
         return False
     for t in tensors:
-        if t is not None and ((type(t) is not Tensor and type(t) is not Parameter) or _functorch.is_legacy_batchedtensor(t)):
+        if t is not None and type(t) is not Tensor and type(t) is not Parameter:
             return False
-    return (not _symbolic_trace._is_fx_tracing_flag and _python_dispatch._get_current_dispatch_mode() is None
-            and _functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
+    return not _symbolic_trace._is_fx_tracing_flag and _python_dispatch._get_current_dispatch_mode() is None
+
+
+def plain_eager(*tensors) -> bool:
+    """True when nothing but the autograd engine looks at these tensors' operators: ``ordinary``, and no ``torch.jit``
+    tracing, no functorch transform (vmap, grad, jvp), no forward-mode level, no batched tensor of the vmap that
+    ``is_grads_batched`` runs under (its type is ``Tensor`` as well), no torch-function mode, and no running profiler
+    (it records the registered ops)."""
+    if not ordinary(*tensors):
+        return False
+    for t in tensors:
+        if t is not None and _functorch.is_legacy_batchedtensor(t):
+            return False
+    return (_functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
             and _get_tracing_state() is None and not _is_torch_function_mode_enabled()
             and not profiler._is_profiler_enabled)
 

@@ -134,7 +134,7 @@ def _delta_rule_args(name, q, k, v, g, beta, scale, initial_state, cu_seqlens, c
     return b, t, h, kd, hv, vd, n, flags, float(scale), A_log, dt_bias
 
 
-_plain_eager = _library.plain_eager  # an ordinary tensor outside compile, tracing, transforms and dispatch modes
+_plain_eager = _library.plain_eager  # ordinary tensors outside compile, tracing, transforms and modes
 
 
 _recurrent_noted: set = set()
@@ -180,10 +180,9 @@ def _gdn_call(entry, name, q, k, v, g, beta, scale, initial_state, output_final_
         # Plain eager calls (no compile or fake tensors, no dispatch mode recording ops) run the op's
         # implementation directly, under grad through an autograd function of it: the dispatcher round
         # trip costs more host time than the kernel launches.
-        eager = _plain_eager(q)
-        # the fp16 operand range guard (sorernn_amd/range_guard.py) reads its flag in eager calls only
-        word = _range.before_call(q.device) if eager else None
-        op = _library.chunk_fwd_call if needs_grad else _library.chunk_fwd_impl if eager else _library.chunk_fwd
+        # the fp16 operand range guard (sorernn_amd/range_guard.py) reads its flag in eager calls, whatever watches them
+        word = _range.before_call(q.device) if _library.ordinary(q) else None
+        op = _library.chunk_fwd_call if needs_grad else _library.chunk_fwd_impl if _plain_eager(q) else _library.chunk_fwd
         o, final, _, _ = op(q, k, v, g, beta, initial_state, a_log_in if use_gate_in_kernel else None,
                             dt_bias_in if use_gate_in_kernel else None, cu_seqlens, scale, flags, n,
                             bool(output_final_state), needs_grad)

@@ -3,12 +3,14 @@
 The kernels are replaced by a recorder (the outputs' values are never looked at): plain eager calls must not
 enter the registered op, and every context that looks at operators must see it, as before the direct route.
 """
+import contextlib
+
 import pytest
 import torch
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from sorernn_amd import _lib, library
+from sorernn_amd import _lib, library, ops
 
 
 class Seen(TorchDispatchMode):
@@ -150,6 +152,23 @@ def test_function_modes_and_the_profiler_see_the_op(launches, which):
     launches[1].clear()
     y.sum().backward()
     assert not launches[1]
+
+
+@pytest.mark.parametrize("context", [None, "vmap", "forward_ad", "function_mode", "profiler"])
+def test_range_guard_reads_its_flag_in_every_eager_call(launches, monkeypatch, context):
+    """Also where the call takes the registered op because something watches it."""
+    monkeypatch.setattr(ops, "_check_cuda", lambda name, *t: t[0].device)
+    word = torch.zeros(1, dtype=torch.int32)
+    monkeypatch.setattr(ops._range, "_words", {0: (word, word.numpy())})
+    monkeypatch.setattr(ops._range, "_device_index", lambda d: 0)
+    q, v, g = _x(2, 1, 8, 1, 64, grad=False), _x(1, 8, 1, 64, grad=False), torch.zeros(1, 8, 1)
+    fn = lambda t: ops.chunk_gated_delta_rule(t, t, v, g, g)[0].float().sum()  # noqa: E731
+    around = {"forward_ad": torch.autograd.forward_ad.dual_level, "function_mode": SeenFunctions,
+              "profiler": lambda: torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU])}
+    word[0] = 1
+    with pytest.warns(RuntimeWarning, match="earlier chunked forward"), around.get(context, contextlib.nullcontext)():
+        torch.vmap(fn)(q) if context == "vmap" else fn(q[0])
+    assert word.item() == 0
 
 
 @pytest.mark.parametrize("which", range(4))
