@@ -592,7 +592,7 @@ def _l2norm_first(q: Tensor, n: int, hv: int, vd: int, tokens: int) -> bool:
 def _l2norm_qk(q: Tensor, k: Tensor, eps: float = 1e-12) -> tuple[Tensor, Tensor]:
     """``l2norm`` of q and k without grad: plain eager calls go to the kernel directly (one launch for both, no
     dispatcher round trip)."""
-    if not _plain_eager(q):
+    if not _plain_eager(q, k):
         return _library.l2norm_fwd(q, float(eps)), _library.l2norm_fwd(k, float(eps))
     q, k = q.contiguous(), k.contiguous()
     qn, kn = torch.empty_like(q), torch.empty_like(k)

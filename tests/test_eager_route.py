@@ -171,6 +171,21 @@ def test_range_guard_reads_its_flag_in_every_eager_call(launches, monkeypatch, c
     assert word.item() == 0
 
 
+@pytest.mark.parametrize("watched", ["q", "k"])
+def test_qk_norm_looks_at_both_tensors(launches, watched):
+    calls, entered = launches
+
+    class Sub(torch.Tensor):
+        pass
+
+    x = {n: _x(1, 8, 1, 64, grad=False) for n in ("q", "k")}
+    ops._l2norm_qk(**x)
+    assert calls == ["gdn_qk_l2norm_fwd"] and not entered
+    x[watched] = x[watched].as_subclass(Sub)
+    ops._l2norm_qk(**x)
+    assert entered == ["l2norm_fwd"] * 2
+
+
 @pytest.mark.parametrize("which", range(4))
 def test_batched_gradients_loop_over_the_op(launches, which):
     """``is_grads_batched`` and vectorised Jacobians: one launch of the backward per gradient."""
