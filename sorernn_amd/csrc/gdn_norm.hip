@@ -317,9 +317,9 @@ __global__ __launch_bounds__(256) void gated_delta_norm_bwd_vec_kernel(NormBwdPa
           dot += d[e] * x[e];
         }
         dot = group_sum<LPR>(dot) / (float)D;
-        const float c3 = rr * rr * rr * dot;
+        const float c = rr * (rr * dot);  // of the order of d: r^3 alone is subnormal from an rms of 4e12 up
 #pragma unroll
-        for (int e = 0; e < V; ++e) ox[e] = (E)(rr * d[e] - x[e] * c3);
+        for (int e = 0; e < V; ++e) ox[e] = (E)(rr * d[e] - x[e] * rr * c);
       }
       if (r < p.rows) {
         const int64_t at = r * D + li * V;

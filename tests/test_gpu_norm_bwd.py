@@ -56,3 +56,21 @@ def test_norm_backwards_at_tile_edges(dtype, rows, d):
         scale[1] = dy.double().abs() * u_terms * (1 + g.double().abs())
         for i, a, r in zip(pick, gots, refs):
             _check(f"rms {act} gated={gated} grad {i}", a, r, scale[i])
+
+
+@pytest.mark.parametrize("size", [1e-3, 1e10, 1e15, 1e17])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rms_backward_of_large_and_small_rows(dtype, size):
+    """r^3 leaves fp32's range long before the row's sum of squares does. dx = r (du w - n mean(du w n)): the bound is
+    one rounding and 2^-20 of r's largest product, n and the mean of 128 products each of at most |n| <= 12."""
+    gen = torch.Generator().manual_seed(5)
+    x, dy = ((size if i == 0 else 1.0) * torch.randn(33, 128, generator=gen) for i in range(2))
+    x, dy, w = x.to(dtype), dy.to(dtype), torch.randn(128, generator=gen)
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    rr = torch.rsqrt(xr.square().mean(-1, keepdim=True) + 1e-6)
+    ref = torch.autograd.grad(xr * rr * wr, [xr, wr], dy.double())
+    xd, wd = x.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(True)
+    got = torch.autograd.grad(rms_norm_gated(xd, None, wd), [xd, wd], dy.to(DEV))
+    rd, n = rr.detach(), (xr * rr).detach()
+    _check("dx", got[0], ref[0], rd * (dy.double() * w.double()).abs().amax(-1, keepdim=True) * (1 + n.abs().amax()) ** 2)
+    _check("dweight", got[1], ref[1], (dy.double() * n).abs().sum(0))
