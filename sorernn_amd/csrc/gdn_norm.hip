@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void gated_delta_norm_bwd_vec_kernel(NormBwdPa
   for (int64_t r0 = wave * RPW * U; r0 < p.rows; r0 += nwaves * RPW * U) {
     VE xv[U], dv[U], gv[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {  // rows past the end: zeros, so that they add nothing to dw and db
+    for (int u = 0; u < U; ++u) {  // rows past the end: zeros, so that they add nothing to db
       const int64_t r = r0 + u * RPW + sub;
       xv[u] = dv[u] = gv[u] = VE{};
       if (r < p.rows) {
@@ -295,7 +295,8 @@ __global__ __launch_bounds__(256) void gated_delta_norm_bwd_vec_kernel(NormBwdPa
 #pragma unroll
         for (int e = 0; e < V; ++e) ox[e] = (E)((d[e] - x[e] * dot) * inv);
       } else {
-        const float rr = 1.f / sqrtf(ss / (float)D + p.eps);
+        // 0 past the end: with eps = 0 a row of zeros has r = inf, and its 0 * inf would reach dw
+        const float rr = r < p.rows ? 1.f / sqrtf(ss / (float)D + p.eps) : 0.f;
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           const float n = x[e] * rr;

@@ -74,3 +74,24 @@ def test_rms_backward_of_large_and_small_rows(dtype, size):
     rd, n = rr.detach(), (xr * rr).detach()
     _check("dx", got[0], ref[0], rd * (dy.double() * w.double()).abs().amax(-1, keepdim=True) * (1 + n.abs().amax()) ** 2)
     _check("dweight", got[1], ref[1], (dy.double() * n).abs().sum(0))
+
+
+@pytest.mark.parametrize("rows", [1, 31, 33, 1025])
+@pytest.mark.parametrize("gated", [True, False])
+def test_rms_backward_without_eps(rows, gated):
+    """eps = 0: the rows that fill the last tile up take no part in the parameter gradients."""
+    gen = torch.Generator().manual_seed(rows)
+    x, g, dy = (torch.randn(rows, 128, generator=gen) for _ in range(3))
+    w, b = torch.randn(128, generator=gen), torch.randn(128, generator=gen)
+    ref_in = [t.double().requires_grad_(True) for t in (x, w, b)]
+    u = ref_in[0] * torch.rsqrt(ref_in[0].square().mean(-1, keepdim=True)) * ref_in[1] + ref_in[2]
+    act = F.silu(g.double()) if gated else torch.ones(1).double()
+    ref = torch.autograd.grad(u * act, ref_in, dy.double())
+    dev = [t.to(DEV).requires_grad_(True) for t in (x, w, b)]
+    got = torch.autograd.grad(rms_norm_gated(dev[0], g.to(DEV) if gated else None, dev[1], dev[2], eps=0.0), dev, dy.to(DEV))
+    n = (x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True))).abs()
+    du = (dy.double() * act).abs()
+    _check("dx", got[0], ref[0], n.amax() ** 2 * (du * w.double().abs()).amax(-1, keepdim=True)
+           * torch.rsqrt(x.double().square().mean(-1, keepdim=True)))
+    _check("dweight", got[1], ref[1], (du * n).sum(0))
+    _check("dbias", got[2], ref[2], du.sum(0))
