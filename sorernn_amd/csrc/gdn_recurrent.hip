@@ -136,6 +136,7 @@ struct RowVec {
 };
 
 constexpr int kShortTokens = 4;
+constexpr float kGrowth = 13.8f;  // log of 2^20
 
 // The recurrence of a few tokens (a decode call, a draft of two or three): one pass over at most G = 4 tokens at a
 // time, all their loads issued at once. Columns of the state are independent (column j needs only S[:, j]), so
@@ -253,6 +254,9 @@ __global__ __launch_bounds__(256) void gated_delta_recurrent_short_kernel(RecPar
 // and Q S as they stand. Helper waves prepare what does not depend on S, ahead of them: waves 4 and 5 the k and
 // q rows of the tokens two steps ahead (normalised, fp32, in LDS; their loads a step earlier still), wave 6 the
 // decays and the k.k coefficients of the next step, wave 7 its q.k coefficients. One barrier per 16 tokens.
+//   The model's decays are at most 1, but the call takes any g. A product of decays past fp32's range would meet a zero
+// (a zero state, a zero product of rows) as 0 * inf, and past a small state it overflows where the state itself does
+// not. A sequence with 16 tokens whose positive log decays add up to more than kGrowth takes a token a step.
 //   Rounding: the decays' products are formed in 64 bits (by the helpers) and rounded once, a step's update and
 // what earlier tokens take from x are summed apart and added once, and the sums over K run in partial sums, so
 // that the error against 64 bits is that of the token-by-token kernel before it (fp32, 500 tokens of K = 128: o
@@ -270,6 +274,7 @@ __global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recur
   __shared__ __align__(16) float cm[2][C * P], pm[2][C * P];  // cm[j][t] = beta_t E_tj k_t.k_j, pm[t][j] = E_tj q_t.k_j
   __shared__ __align__(16) float bs[2][C], es[2][C], ed[2][C];  // beta_t, e_t, E_15,j
   __shared__ __align__(16) float xs[4][C * P];                  // per state wave: x by column
+  __shared__ int tokens;                                        // a step's tokens
   const int t = threadIdx.x, lane = t % kWave, w = __builtin_amdgcn_readfirstlane(t / kWave);
   const int li = lane % 16, g = lane / 16;
   constexpr int kSlices = VD / 64;
@@ -284,12 +289,31 @@ __global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recur
     bos = n * p.T;
     eos = bos + p.T;
   }
-  const int steps = (int)((eos - bos + C - 1) / C);
+  // Tokens a step: 16, or 1 where the decays of 16 tokens grow too far (a gate formed in the kernel is never positive).
+  // Each helper wave looks at all of the sequence's log decays by itself, under its first loads: no exchange, no barrier.
+  auto step_tokens = [&]() {
+    bool up = false;
+    auto raw_g = [&](int64_t at) { return at < eos ? load_raw32(p.g, p.dg, at * p.HV + hv) : 0u; };
+    auto look = [&](uint32_t raw) {  // at 64 tokens, a step's in 16 lanes
+      const float x = fmaxf(raw32_to_f32(raw, p.dg), 0.f);
+      if (__any(x > 0.f)) up |= group_sum<C>(x) > kGrowth;
+    };
+    if (!(p.flags & GDN_FLAG_GATE_IN_KERNEL)) {
+      look(raw_g(bos + lane));
+      for (int64_t at = bos + kWave; at < eos; at += 4 * kWave) {
+        uint32_t raw[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) raw[u] = raw_g(at + u * kWave + lane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) look(raw[u]);
+      }
+    }
+    return __any(up) ? 1 : C;
+  };
   auto mm = [](float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); };
   auto ld4 = [](const float* x) { return *reinterpret_cast<const f32x4*>(x); };
-  auto tok = [&](int i, int c) {  // token c of step i; past the end the last token (its values are cleared)
-    const int64_t at = bos + (int64_t)i * C + c;
-    return at < eos ? at : eos - 1;
+  auto tok = [&](int64_t first, int c) {  // token c from `first` on; past the end the last token (its values are cleared)
+    return first + c < eos ? first + c : eos - 1;
   };
 
   if (w < 4) {
@@ -303,23 +327,25 @@ __global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recur
     const E* __restrict__ vp = static_cast<const E*>(p.v) + (int64_t)hv * VD + col;
     E* __restrict__ op = static_cast<E*>(p.o) + (int64_t)hv * VD + col;
     E vr[4];
-    if (steps > 0) {
+    if (bos < eos) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vr[r] = vp[tok(0, 4 * g + r) * p.HV * VD];
+      for (int r = 0; r < 4; ++r) vr[r] = vp[tok(bos, 4 * g + r) * p.HV * VD];
     }
     __syncthreads();
+    const int L = __builtin_amdgcn_readfirstlane(tokens), steps = (int)((eos - bos + L - 1) / L);
     __syncthreads();
     for (int i = 0; i < steps; ++i) {
       const float* kl = kt[i % 3];
       const float* ql = qt[i % 3];
       const int li = opaque_int(lane % 16), g = opaque_int(lane / 16);  // addresses made here, not kept across steps
-      const int b = i & 1, left = (int)(eos - bos - (int64_t)i * C < C ? eos - bos - (int64_t)i * C : C);
+      const int64_t first = bos + (int64_t)i * L;
+      const int b = i & 1, left = (int)(eos - first < L ? eos - first : L);
       float v[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] = 4 * g + r < left ? (float)vr[r] : 0.f;
       if (i + 1 < steps) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) vr[r] = vp[tok(i + 1, 4 * g + r) * p.HV * VD];
+        for (int r = 0; r < 4; ++r) vr[r] = vp[tok(first + L, 4 * g + r) * p.HV * VD];
       }
       f32x4 yp[NP]{}, zp[NP]{};  // K S and Q S in partial sums: lane (g, i) column i, tokens 4g + r
 #pragma unroll
@@ -398,7 +424,7 @@ __global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recur
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (4 * g + r < left) op[(bos + (int64_t)i * C + 4 * g + r) * p.HV * VD] = (E)o[r];
+        if (4 * g + r < left) op[(first + 4 * g + r) * p.HV * VD] = (E)o[r];
       __syncthreads();
     }
     if (p.ht) {
@@ -415,14 +441,15 @@ __global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recur
     const E* __restrict__ qp = static_cast<const E*>(p.q) + (int64_t)h * KD + pos;
     const bool l2 = p.flags & GDN_FLAG_QK_L2NORM;
     VK kr{}, qr{};
-    auto load = [&](int i) {
-      kr = *reinterpret_cast<const VK*>(kp + tok(i, row) * p.H * KD);
-      qr = *reinterpret_cast<const VK*>(qp + tok(i, row) * p.H * KD);
+    auto load = [&](int64_t first) {
+      kr = *reinterpret_cast<const VK*>(kp + tok(first, row) * p.H * KD);
+      qr = *reinterpret_cast<const VK*>(qp + tok(first, row) * p.H * KD);
     };
-    if (steps > 0) load(0);
+    if (bos < eos) load(bos);
+    const int L = step_tokens(), steps = (int)((eos - bos + L - 1) / L);
     for (int i = -2; i < steps; ++i) {
       if (i + 2 < steps) {  // F.normalize: x / max(|x|, 1e-12); q times the scale; zeros past the end
-        const bool live = bos + (int64_t)(i + 2) * C + row < eos;
+        const bool live = row < L && bos + (int64_t)(i + 2) * L + row < eos;
         float kf[R], qf[R], kk = 0.f, qq = 0.f;
 #pragma unroll
         for (int e = 0; e < R; ++e) {
@@ -443,30 +470,32 @@ __global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recur
           *reinterpret_cast<f32x4*>(kl + e) = f32x4{kf[e] * ks, kf[e + 1] * ks, kf[e + 2] * ks, kf[e + 3] * ks};
           *reinterpret_cast<f32x4*>(ql + e) = f32x4{qf[e] * qs, qf[e + 1] * qs, qf[e + 2] * qs, qf[e + 3] * qs};
         }
-        if (i + 3 < steps) load(i + 3);
+        if (i + 3 < steps) load(bos + (int64_t)(i + 3) * L);
       }
       __syncthreads();
     }
   } else {  // coefficients of the next step: wave 6 k.k (with beta), wave 7 q.k
     uint32_t graw = 0, braw = 0;
-    auto load = [&](int i) {
-      graw = load_raw32(p.g, p.dg, tok(i, li) * p.HV + hv);
-      if (w == 6) braw = load_raw32(p.beta, p.db, tok(i, li) * p.HV + hv);
+    auto load = [&](int64_t first) {
+      graw = load_raw32(p.g, p.dg, tok(first, li) * p.HV + hv);
+      if (w == 6) braw = load_raw32(p.beta, p.db, tok(first, li) * p.HV + hv);
     };
     const float neg_a = p.flags & GDN_FLAG_GATE_IN_KERNEL ? -expf(p.A_log[hv]) : 0.f;
     const float dtb = p.flags & GDN_FLAG_GATE_IN_KERNEL ? p.dt_bias[hv] : 0.f;
-    if (steps > 0) load(0);
+    if (bos < eos) load(bos);
+    const int L = step_tokens(), steps = (int)((eos - bos + L - 1) / L);
+    if (t == 6 * kWave) tokens = L;
     __syncthreads();
     for (int i = 0; i <= steps; ++i) {  // step i, while the state waves work on step i - 1
       if (i < steps) {
         const int b = i & 1;
-        const bool live = bos + (int64_t)i * C + li < eos;
+        const bool live = li < L && bos + (int64_t)i * L + li < eos;
         float gv = raw32_to_f32(graw, p.dg), bv = raw32_to_f32(braw, p.db);
         if (p.flags & GDN_FLAG_GATE_IN_KERNEL) gv = neg_a * softplus_f32(gv + dtb);
         if (p.flags & GDN_FLAG_BETA_SIGMOID) bv = sigmoid_f32(bv);
         const double av = live ? exp((double)gv) : 1.0;  // decays in 64 bits up to the products that leave here
         bv = live ? bv : 0.f;
-        if (i + 1 < steps) load(i + 1);
+        if (i + 1 < steps) load(bos + (int64_t)(i + 1) * L);
         const float* kl = kt[i % 3] + li * KP + 4 * g;
         const float* rl = w == 6 ? kl : qt[i % 3] + li * KP + 4 * g;
         f32x4 dp[8]{};  // lane (g, j): rows (tokens) 4g + r, column (earlier token) j

@@ -91,3 +91,38 @@ def test_nan_reaches_only_later_tokens_of_its_head(t, bad, where):
     assert not torch.isfinite(o[0, bad, 1]).any()
     if where == "q":
         assert torch.isfinite(o[0, bad + 1:]).all() and torch.isfinite(st).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("t", [3, 16, 23, 40])
+@pytest.mark.parametrize("kd,vd", [(128, 128), (64, 64), (128, 64), (64, 128)])
+def test_decays_above_one(kd, vd, t, dtype):
+    """Nine log decays of 10, then nine of -10, of tiny states and values: the products of the decays leave fp32's range, the
+    states stay in it. Error of a token: T sums of K terms, sqrt(K) T 2^-24 < 2^-15 of its state's largest column."""
+    q, k, v, _, beta, h0 = _inputs(1, t, 2, 2, kd, vd, 1, dtype, t)
+    g = torch.zeros(1, t, 2)
+    g[:, 2:11], g[:, 11:20] = 10.0, -10.0
+    v = 1e-10 * v
+    o, st = fused_recurrent_gated_delta_rule(*(x.to(DEV) for x in (q, k, v, g, beta)), initial_state=1e-10 * h0.to(DEV),
+                                             output_final_state=True)
+    s, scale = 1e-10 * h0.double(), kd**-0.5
+    for i in range(t):
+        s = s * g[:, i].double().exp()[..., None, None]
+        ki, qi = k[:, i].double(), q[:, i].double()
+        d = beta[:, i].double()[..., None] * (v[:, i].double() - (s * ki[..., None]).sum(-2))
+        s = s + ki[..., None] * d[..., None, :]
+        ref, top = scale * (s * qi[..., None]).sum(-2), s.norm(dim=-2).amax(-1, keepdim=True)
+        err, bound = (o[:, i].double().cpu() - ref).abs(), 2.0**-15 * scale * top + HALF_ULP[dtype] * ref.abs() * 1.01
+        assert (err <= bound).all(), f"token {i}: {(err / bound).max().item():.2f} of the bound"
+    assert ((st.double().cpu() - s).abs() <= 2.0**-15 * s.norm(dim=-2, keepdim=True).amax(-1, keepdim=True)).all()
+
+
+@pytest.mark.parametrize("t", [4, 16, 40])
+def test_decays_above_one_leave_a_zero_state(t):
+    q, k, v, _, beta, _ = _inputs(2, t, 2, 2, 128, 128, 2, torch.bfloat16, t)
+    v[:, 7:] = 0  # the state is zero from the -inf on
+    g = torch.full((2, t, 2), 20.0)
+    g[:, 7:8] = -float("inf")
+    g[:, :7] = 0
+    o, st = fused_recurrent_gated_delta_rule(*(x.to(DEV) for x in (q, k, v, g, beta)), output_final_state=True)
+    assert torch.isfinite(o).all() and not o[:, 7:].any() and (t < 8 or not st.any())
