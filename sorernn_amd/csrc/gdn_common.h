@@ -77,9 +77,16 @@ __device__ __forceinline__ float silu_fast(float x) {
   return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
 }
 
-// The logistic function by the same two instructions (for gradients rounded to a 16-bit type).
-__device__ __forceinline__ float sigmoid_fast(float x) {
-  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
+// The logistic function for the backwards of 16-bit rows, whose fp32 parameter gradients carry it: v_exp_f32 of
+// -x log2(e), times what rounding that product to fp32 left out, and a reciprocal with one Newton step. Mean square
+// error against 64 bits, in 2^-24, and that of sigmoid_f32: 0.70 and 0.73 within +-2, 0.86 and 1.8 at -6 to -2, 0.89
+// and 18.7 at -60 to -20, without a bias. The conv backward of 16,384 x 2,048 in bf16 takes 50 us with it, 60 with
+// sigmoid_f32.
+__device__ __forceinline__ float sigmoid_comp(float x) {
+  const float t = x * -1.44269502f, lo = fmaf(x, -1.925963e-8f, fmaf(x, -1.44269502f, -t));
+  const float d = fminf(fmaf(__builtin_amdgcn_exp2f(t), fmaf(lo, 0.693147182f, 1.f), 1.f), 1e38f);  // finite: no inf * 0
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.f), r, r);
 }
 
 // ---------------------------------------------------------------- wave reductions

@@ -465,13 +465,12 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_bwd_kernel(ConvBwdPara
 // take consecutive token segments of the same 256 channels, so the segments' overlapping rows meet in the
 // cache and one row of dw/dbias partial sums leaves per workgroup (added over the waves in LDS) instead of
 // one per segment. 4 channels and not 8, so that the per-channel state (weights, window, pending dx, dw: 17
-// values) leaves room for 4 waves per SIMD. 16,384 tokens x 2,048 channels in bf16, 24 documents: 49 us (4.1 TB/s) against 146
+// values) leaves room for 4 waves per SIMD. 16,384 tokens x 2,048 channels in bf16, 24 documents: 50 us (4.0 TB/s) against 146
 // with one channel per thread (the kernel above, kept for other W, C and alignments).
 template <typename E>
 __global__ __launch_bounds__(256) void gated_delta_conv1d_bwd_vec_kernel(ConvBwdParams p, int tt) {
   constexpr int W = 4, V = 4, G = 4;
   typedef E VE __attribute__((ext_vector_type(V)));
-  constexpr bool kFast = sizeof(E) == 2;  // results rounded to 16 bits: sigmoid from v_exp_f32 / v_rcp_f32
   __shared__ __align__(16) float red[4][W + 1][kWave * V];
   const int lane = threadIdx.x % kWave, wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const unsigned c0 = (blockIdx.x * kWave + lane) * V;
@@ -565,7 +564,7 @@ __global__ __launch_bounds__(256) void gated_delta_conv1d_bwd_vec_kernel(ConvBwd
           for (int i = 0; i < W - 1; ++i) z += w[e][i] * win[i][e];
           dz[e] = (float)dv[g][e];
           if (p.act == GDN_ACT_SILU) {
-            const float sg = kFast ? sigmoid_fast(z) : sigmoid_f32(z);
+            const float sg = sizeof(E) == 2 ? sigmoid_comp(z) : sigmoid_f32(z);
             dz[e] *= sg * (1.f + z * (1.f - sg));
           }
         }

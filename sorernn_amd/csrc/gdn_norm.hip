@@ -244,7 +244,7 @@ template <typename E, int V, int LPR, int MODE>
 __global__ __launch_bounds__(256) void gated_delta_norm_bwd_vec_kernel(NormBwdParams p) {
   typedef E VE __attribute__((ext_vector_type(V)));
   constexpr int D = V * LPR, RPW = kWave / LPR, U = MODE == 0 ? 4 : 2;
-  constexpr bool kGate = MODE >= 2, kFast = sizeof(E) == 2;  // outputs rounded to 16 bits: fast sigmoid
+  constexpr bool kGate = MODE >= 2;
   const int lane = threadIdx.x % kWave, sub = lane / LPR, li = lane % LPR;
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) / kWave;
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) void gated_delta_norm_bwd_vec_kernel(NormBwdPa
             const float g = (float)gv[u][e], un = n * wv[e] + bv[e];
             float act = g, dact = 1.f;
             if (MODE == 2) {
-              const float sg = kFast ? sigmoid_fast(g) : sigmoid_f32(g);
+              const float sg = sizeof(E) == 2 ? sigmoid_comp(g) : sigmoid_f32(g);
               act = g * sg;
               dact = sg * (1.f + g * (1.f - sg));
             }

@@ -95,3 +95,19 @@ def test_rms_backward_without_eps(rows, gated):
            * torch.rsqrt(x.double().square().mean(-1, keepdim=True)))
     _check("dweight", got[1], ref[1], (du * n).sum(0))
     _check("dbias", got[2], ref[2], du.sum(0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_rms_parameter_gradients_of_saturated_gates(dtype):
+    """The fp32 parameter gradients carry the gate's activation in fp32, whatever type the rows have: terms of one size
+    over 128 gates. A gate's activation is off by up to 40 units (expf's argument reduction at -50), by a third of that in
+    the mean square and either way: 14 / sqrt(128) units for the sum, 5 are allowed. A bias would add up to all of them."""
+    g = (-50 + torch.arange(128) / 32).repeat(64)[:, None].expand(-1, 128).to(dtype).contiguous()
+    dy = (0.5 * torch.exp(-48 - g.float())).to(dtype)
+    x = torch.randn(g.shape, generator=torch.Generator().manual_seed(1)).to(dtype)
+    b = torch.zeros(128, device=DEV, requires_grad=True)
+    y = rms_norm_gated(x.to(DEV), g.to(DEV), torch.ones(128, device=DEV), b)
+    (got,) = torch.autograd.grad(y, b, dy.to(DEV))
+    ref = (dy.double() * F.silu(g.double())).sum(0)
+    err = ((got.double().cpu() - ref) / ref).abs().max().item()
+    assert err <= 5 * 2.0**-24, err * 2**24
