@@ -248,6 +248,13 @@ GDN_API int gdn_qk_l2norm_fwd(const void* q, const void* k, void* q_out, void* k
                               float eps, void* stream);
 
 /*
+ * The rows that the chunk forward makes of bf16 q and k under GDN_FLAG_QK_L2NORM, bit for bit: gdn_chunk_fwd of them
+ * without the flag equals gdn_chunk_fwd of q and k with it. D is 64 or 128, the pointers 16-byte aligned.
+ */
+GDN_API int gdn_qk_l2norm_chunk_fwd(const void* q, const void* k, void* q_out, void* k_out, int64_t rows, int64_t D,
+                                    void* stream);
+
+/*
  * Gated RMSNorm: y = x * rsqrt(mean(x^2) + eps) * weight (+ bias) * act(gate), per row of D.
  * Replaces FLA rms_norm_gated(o, gate, weight, None, activation="swish", eps) at
  * sore/model/gdn.py:182-186 and o_norm(o) * F.silu(gate) at gdn.py:188 (RMSNorm:

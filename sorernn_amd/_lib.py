@@ -50,6 +50,7 @@ SIGNATURES = {
     "gdn_causal_conv1d_fwd": [_P] * 7 + [_I64] * 5 + [_INT, _INT, _U, _P],
     "gdn_l2norm_fwd": [_P, _P, _I64, _I64, _INT, _F, _P],
     "gdn_qk_l2norm_fwd": [_P, _P, _P, _P, _I64, _I64, _INT, _F, _P],
+    "gdn_qk_l2norm_chunk_fwd": [_P, _P, _P, _P, _I64, _I64, _P],
     "gdn_rms_norm_gated_fwd": [_P] * 5 + [_I64, _I64, _INT, _F, _INT, _P],
     "gdn_causal_conv1d_bwd": [_P] * 6 + [_I64] * 5 + [_INT, _INT, _U] + [_P] * 5 + [_SZ, _P],
     "gdn_causal_conv1d_bwd_workspace_size": [_I64] * 4,

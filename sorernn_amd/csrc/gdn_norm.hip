@@ -19,7 +19,7 @@ struct NormParams {
   int64_t rows, D;
   int dt, act;
   float eps;
-  int mode;   // 0 = L2 norm, 1 = (gated) RMSNorm
+  int mode;   // 0 = L2 norm, 1 = (gated) RMSNorm, 2 = L2 norm as the chunk kernels form it (vector path only)
   int split;  // RMSNorm with a gate: the norm (w, bias) and act(gate) each rounded before their product
   const void* x2;  // a second tensor of the same rows, normalised by the blocks with blockIdx.y = 1
   void* y2;
@@ -113,7 +113,9 @@ __global__ __launch_bounds__(256) void gated_delta_norm_v8_kernel(NormParams p) 
         ss += xf[e] * xf[e];
       }
       ss = group_sum<LPR>(ss);
-      const float scale = p.mode == 0 ? 1.f / fmaxf(sqrtf(ss), p.eps) : __builtin_amdgcn_rsqf(ss / (float)p.D + p.eps);
+      const float scale = p.mode == 0   ? 1.f / fmaxf(sqrtf(ss), p.eps)
+                          : p.mode == 2 ? __builtin_amdgcn_rsqf(fmaxf(ss, 1e-24f))  // as l2norm_row_chunks, its sums too
+                                        : __builtin_amdgcn_rsqf(ss / (float)p.D + p.eps);
       V8 yv;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -469,6 +471,18 @@ extern "C" int gdn_qk_l2norm_fwd(const void* q, const void* k, void* q_out, void
   }
   NormParams p{q, nullptr, nullptr, nullptr, q_out, rows, D, dtype, GDN_ACT_NONE, eps, 0, 0, k, k_out};
   return launch_norm(p, stream, "gated_delta_norm_kernel(qk l2)");
+}
+
+extern "C" int gdn_qk_l2norm_chunk_fwd(const void* q, const void* k, void* q_out, void* k_out, int64_t rows, int64_t D,
+                                       void* stream) {
+  const uintptr_t al = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                       reinterpret_cast<uintptr_t>(q_out) | reinterpret_cast<uintptr_t>(k_out);
+  if (!q || !k || !q_out || !k_out || rows < 0 || (D != 64 && D != 128) || (al & 15)) {
+    gdn_internal_set_error("gdn_qk_l2norm_chunk_fwd: bad arguments (rows=%lld D=%lld)", (long long)rows, (long long)D);
+    return GDN_ERR_INVALID;
+  }
+  NormParams p{q, nullptr, nullptr, nullptr, q_out, rows, D, GDN_DTYPE_BF16, GDN_ACT_NONE, 0.f, 2, 0, k, k_out};
+  return launch_norm(p, stream, "gated_delta_norm_kernel(chunk qk l2)");
 }
 
 extern "C" int gdn_rms_norm_gated_fwd(const void* x, const void* gate, const float* weight, const float* bias, void* y,

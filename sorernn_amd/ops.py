@@ -170,10 +170,8 @@ def _gdn_call(entry, name, q, k, v, g, beta, scale, initial_state, output_final_
             "require grad); run under torch.no_grad() or detach the inputs"
         )
     q_raw, k_raw = q, k
-    if (entry == "gdn_chunk_fwd" and (flags & _lib.FLAG_QK_L2NORM) and not needs_grad
-            and _l2norm_first(q, n, hv, vd, b * t)):
-        q, k = _l2norm_qk(q, k)
-        flags &= ~_lib.FLAG_QK_L2NORM
+    if entry == "gdn_chunk_fwd" and (flags & _lib.FLAG_QK_L2NORM) and not needs_grad:
+        q, k, flags = _chunk_qk(q, k, n, hv, vd, b * t, flags)
     if entry == "gdn_chunk_fwd":
         # the torch.library op (sorernn::chunk_gated_delta_rule_fwd): traceable by torch.compile, with
         # the backward registered on it; with grad it also keeps the per-chunk states for the backward.
@@ -328,9 +326,8 @@ def chunk_gated_delta_rule_gated_norm(
         raise ValueError(f"{name}: norm_weight must be [{vd}] (got {tuple(norm_weight.shape)})")
     word = _range.before_call(q.device)
     q_raw, k_raw = q, k
-    if (flags & _lib.FLAG_QK_L2NORM) and _l2norm_first(q, n, hv, vd, b * t):
-        q, k = _l2norm_qk(q, k)
-        flags &= ~_lib.FLAG_QK_L2NORM
+    if flags & _lib.FLAG_QK_L2NORM:
+        q, k, flags = _chunk_qk(q, k, n, hv, vd, b * t, flags)
     q, k, v, g, beta, gate = (x.contiguous() for x in (q, k, v, g, beta, gate))
     w = norm_weight.float().contiguous()
     h0 = None if initial_state is None else initial_state.float().contiguous()
@@ -567,6 +564,14 @@ def qkv_causal_conv1d(x: Tensor, weight: Tensor, qk_dim: int, v_dim: int, head_d
 _cu_count: dict = {}
 
 
+def _cus(x: Tensor) -> int:
+    dev = x.get_device()
+    cus = _cu_count.get(dev)
+    if cus is None:
+        cus = _cu_count[dev] = torch.cuda.get_device_properties(dev).multi_processor_count
+    return cus
+
+
 def _l2norm_first(q: Tensor, n: int, hv: int, vd: int, tokens: int) -> bool:
     """Whether an inference call with use_qk_l2norm_in_kernel normalises q and k by the row kernel
     before the chunk kernels (which then run without the flag) instead of inside them.
@@ -578,15 +583,35 @@ def _l2norm_first(q: Tensor, n: int, hv: int, vd: int, tokens: int) -> bool:
     call in the kernels / first, 16 heads of 128: 1 x 512 tokens 32.4 / 34.7 us, 1 x 1000 49.7 / 41.6, 2 x 4096
     161 / 125, 3 x 4096 165 / 149, 4 x 4096 172 / 176, 1 x 16384 589 / 380; of 64: 1 x 1000 32.8 / 34.1, 2 x 4096
     98 / 89, 4 x 2048 57.7 / 59.5."""
-    dev = q.get_device()
-    cus = _cu_count.get(dev)
-    if cus is None:
-        cus = _cu_count[dev] = torch.cuda.get_device_properties(dev).multi_processor_count
     kd = q.shape[3]
-    rounds = n * hv * max(1, vd // 32) / cus
+    rounds = n * hv * max(1, vd // 32) / _cus(q)
     per_step = 0.6 if rounds > 1 else 0.9 if kd >= 128 else 0.35
     saved = per_step * tokens / (64 * max(1, n)) * max(1.0, rounds)
     return saved > 3 + 8 * tokens * hv * kd / 5.2e6 + 4  # hv: q/k heads are at most as many
+
+
+def _chunk_qk(q: Tensor, k: Tensor, n: int, hv: int, vd: int, tokens: int, flags: int) -> tuple[Tensor, Tensor, int]:
+    """q, k and the flags of an inference call that asks for the q/k norm: normalised here and the flag cleared where
+    ``_l2norm_first`` says so, else as they are.
+
+    Where the state kernel leaves half the CUs idle and its sequences have 2,048 tokens or more, the rows are
+    ``l2norm``'s, whose IEEE root and quotient can round to the next bf16. In other calls the choice of the route does
+    not change the result: they are bit for bit the rows that the chunk kernels make, and calls that something watches,
+    or whose rows are not 16-byte aligned, keep the norm in the kernels."""
+    if not _l2norm_first(q, n, hv, vd, tokens):
+        return q, k, flags
+    if 2 * n * hv * max(1, vd // 32) <= _cus(q) and tokens >= 2048 * n:
+        q, k = _l2norm_qk(q, k)
+        return q, k, flags & ~_lib.FLAG_QK_L2NORM
+    if not _plain_eager(q, k):
+        return q, k, flags
+    qc, kc = q.contiguous(), k.contiguous()
+    if (qc.data_ptr() | kc.data_ptr()) & 15:
+        return q, k, flags
+    qn, kn = torch.empty_like(qc), torch.empty_like(kc)
+    _lib.call("gdn_qk_l2norm_chunk_fwd", qc.data_ptr(), kc.data_ptr(), qn.data_ptr(), kn.data_ptr(),
+              qc.numel() // qc.shape[3], qc.shape[3], _lib.stream_of(qc))
+    return qn, kn, flags & ~_lib.FLAG_QK_L2NORM
 
 
 def _l2norm_qk(q: Tensor, k: Tensor, eps: float = 1e-12) -> tuple[Tensor, Tensor]:

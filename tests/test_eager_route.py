@@ -186,6 +186,18 @@ def test_qk_norm_looks_at_both_tensors(launches, watched):
     assert entered == ["l2norm_fwd"] * 2
 
 
+def test_watched_chunk_calls_keep_the_qk_norm_in_the_kernels(launches, monkeypatch):
+    calls, _ = launches
+    monkeypatch.setattr(ops, "_l2norm_first", lambda *a: True)
+    monkeypatch.setattr(ops, "_cus", lambda x: 256)
+    x = torch.randn(1, 1000, 16, 128).bfloat16()
+    q, k, flags = ops._chunk_qk(x, x, 1, 16, 128, 1000, 7)
+    assert flags == 7 & ~_lib.FLAG_QK_L2NORM and calls == ["gdn_qk_l2norm_chunk_fwd"]
+    with SeenFunctions():
+        q, k, flags = ops._chunk_qk(x, x, 1, 16, 128, 1000, 7)
+    assert flags == 7 and q is x and k is x and len(calls) == 1
+
+
 @pytest.mark.parametrize("which", range(4))
 def test_batched_gradients_loop_over_the_op(launches, which):
     """``is_grads_batched`` and vectorised Jacobians: one launch of the backward per gradient."""
