@@ -126,3 +126,26 @@ def test_decays_above_one_leave_a_zero_state(t):
     g[:, :7] = 0
     o, st = fused_recurrent_gated_delta_rule(*(x.to(DEV) for x in (q, k, v, g, beta)), output_final_state=True)
     assert torch.isfinite(o).all() and not o[:, 7:].any() and (t < 8 or not st.any())
+
+
+@pytest.mark.parametrize("n,t", [(15, 4), (15, 5), (16, 6), (16, 7), (31, 6), (32, 8), (32, 9)])
+def test_both_sides_of_the_few_token_lines(n, t):
+    """16 heads of 128: the line lies at 4 tokens, at 6 from 16 sequences up and at 8 from 32 up."""
+    q, k, v, g, beta, h0 = _inputs(n, t, 16, 16, 128, 128, n, torch.bfloat16, 100 * n + t)
+    o, st = fused_recurrent_gated_delta_rule(*(x.to(DEV) for x in (q, k, v, g, beta)), initial_state=h0.to(DEV),
+                                             output_final_state=True)
+    o_ref, st_ref = recurrent_gated_delta_rule(*(x.double() for x in (q, k, v, g, beta)), 128**-0.5, h0.double(), True)
+    _check(o, st, o_ref.double(), st_ref.double(), torch.bfloat16)
+
+
+@pytest.mark.parametrize("long", [65, 193, 194])
+def test_one_long_sequence_among_single_tokens(long):
+    """64 packed sequences, 63 of one token: the mean length picks the kernel (193 + 63 is 4 tokens a sequence).
+    The decays forget: a state holds the rounding of some dozen tokens, and the module's bound serves 194 as well."""
+    lens = [1] * 40 + [long] + [1] * 23
+    q, k, v, g, beta, h0 = _inputs(1, sum(lens), 2, 2, 128, 128, 64, torch.bfloat16, long)
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()])
+    o, st = fused_recurrent_gated_delta_rule(*(x.to(DEV) for x in (q, k, v, g, beta)), initial_state=h0.to(DEV),
+                                             output_final_state=True, cu_seqlens=cu.to(DEV), cu_seqlens_cpu=cu)
+    o_ref, st_ref = recurrent_gated_delta_rule(*(x.double() for x in (q, k, v, g, beta)), 128**-0.5, h0.double(), True, cu_seqlens=cu)
+    _check(o, st, o_ref.double(), st_ref.double(), torch.bfloat16)
