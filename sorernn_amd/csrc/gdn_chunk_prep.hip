@@ -59,7 +59,7 @@ __device__ __forceinline__ bool prep_locate(const ChunkPrepParams& p, int64_t it
 //           F[rt][s] = K[16rt + i][32s + 8g .. +7] (lane (g, i)), the A operand of row tile rt and
 //           equally the B operand of column tile rt; rows past the chunk read as zeros.
 //   gates:  in-chunk cumsum (DPP scan) into LDS; the L2 norm of the k rows (when asked) in
-//           registers, summed in the order l2norm_row_chunk sums, so the rows are bitwise the ones
+//           registers, summed in the order l2norm_row_chunks sums, so the rows are bitwise the ones
 //           the state kernel normalises.
 //   Gram:   the diagonal tiles K_b K_b^T and, for m < b, K_m K_b^T (40 MFMAs at K = 128). The
 //           accumulator of K_m K_b^T holds A[16b + i][16m + 4g + r] once scaled (k.k is symmetric):

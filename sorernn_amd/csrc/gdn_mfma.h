@@ -196,11 +196,5 @@ __device__ __forceinline__ void l2norm_row_chunks(bf16x8 (&x)[U]) {
     for (int i = 0; i < 8; ++i) x[u][i] = static_cast<bf16>((float)x[u][i] * inv);
   }
 }
-template <int KCH>
-__device__ __forceinline__ bf16x8 l2norm_row_chunk(bf16x8 x) {
-  bf16x8 r[1] = {x};
-  l2norm_row_chunks<KCH>(r);
-  return r[0];
-}
 
 }  // namespace gdn

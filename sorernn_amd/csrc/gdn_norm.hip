@@ -376,7 +376,9 @@ __global__ __launch_bounds__(kParamCols* kParamLanes) void gated_delta_norm_para
   }
 }
 
-constexpr int64_t kNormBwdBlocks = 1024;  // most blocks of the RMS backward: 4 per CU, up to 4096 rows of partial sums
+// Most blocks of the RMS backward: 4 per CU, up to 4096 rows of partial sums. The 132 registers of the gated 16-bit
+// kernels let 3 run on a CU at once, the fourth follows.
+constexpr int64_t kNormBwdBlocks = 1024;
 
 // Launches the vector backward when the rows allow it. `blocks` returns the rows of partial sums (RMS).
 static bool launch_norm_bwd_vec(const NormBwdParams& p, hipStream_t s, int64_t* blocks) {

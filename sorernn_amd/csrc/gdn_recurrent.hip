@@ -260,8 +260,9 @@ __global__ __launch_bounds__(256) void gated_delta_recurrent_short_kernel(RecPar
 //   Rounding: the decays' products are formed in 64 bits (by the helpers) and rounded once, a step's update and
 // what earlier tokens take from x are summed apart and added once, and the sums over K run in partial sums, so
 // that the error against 64 bits is that of the token-by-token kernel before it (fp32, 500 tokens of K = 128: o
-// 1.32e-7 against 1.34e-7, state 8.5e-8 against 9.3e-8). 16-bit outputs take two partial sums instead of four: with
-// them the kernel fits 128 registers and two workgroups a CU (16 sequences of 7 tokens 15.3 us against 18.4).
+// 1.32e-7 against 1.34e-7, state 8.5e-8 against 9.3e-8). 16-bit outputs take two partial sums instead of four, which lets
+// two workgroups run on a CU: 109 registers at K = 64, 128 with 4 spilled at K = 128 (16 sequences of 7 tokens 15.3 us
+// against 18.4).
 //   What bounds it: the 3 K / 4 fp32 MFMAs of a step (K = 128: 96 x 32 cycles a wave) and, for few sequences, the
 // chain of a step (K S, x through LDS, the triangular solve, the update). bf16, 16 heads of 128: 16 sequences of 64
 // tokens 37 us against 194 for the kernel before it (a token at a time, two barriers each); fp32, 2 sequences of
@@ -813,7 +814,8 @@ extern "C" int gdn_recurrent_fwd(const void* q, const void* k, const void* v, co
   // tokens in the short kernel and in the 16-token one: 1 sequence 5.9 / 7.5 / 9.3 / 12.0 and 8.5; 16 sequences
   // 11.1 / 13.8 / 16.6 / 21.7 and 15.3; 64 sequences 27.4 / 32.3 / 40.5 / 55.2 and 42 (heads of 64: 11.3 / 14.8 / 17.8
   // / 22.8 and 17.5). The line is at 4 tokens, at 6 from 512 waves of 64 columns up and at 8 from 1,024 up, where
-  // the state's bytes set the time of either.
+  // the state's bytes set the time of either. The mean length decides, as the host does not read cu_seqlens: one long
+  // sequence among many of one token may take the short kernel, at 0.7 us a token.
   const int64_t tokens = cu_seqlens ? T : B * T, cols = N * HV * V;
   const bool few = tokens <= (cols >= 65536 ? 8 : cols >= 32768 ? 6 : kShortTokens) * N;
   auto go = [&](auto e_tag, auto k_c, auto v_c) {

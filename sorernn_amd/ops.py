@@ -141,10 +141,10 @@ _recurrent_noted: set = set()
 
 
 def _note_recurrent_route(name: str, dtype: torch.dtype) -> None:
-    """Warn once per dtype that non-bf16 q/k/v take the token-by-token kernel (no MFMA)."""
+    """Warn once per dtype that non-bf16 q/k/v take the fp32 recurrent kernel (slower, every product in fp32)."""
     if dtype not in _recurrent_noted:
         _recurrent_noted.add(dtype)
-        warnings.warn(f"{name}: {dtype} q/k/v run on the token-by-token fp32 recurrent kernel, not the chunked "
+        warnings.warn(f"{name}: {dtype} q/k/v run on the fp32 recurrent kernel (16 tokens at a time), not the chunked "
                       "MFMA prefill (bf16 q/k/v only); cast q/k/v to bfloat16 for the chunked path "
                       "(reported once per dtype)", RuntimeWarning, stacklevel=4)
 
@@ -159,7 +159,7 @@ def _gdn_call(entry, name, q, k, v, g, beta, scale, initial_state, output_final_
         use_qk_l2norm_in_kernel, use_beta_sigmoid_in_kernel, use_gate_in_kernel, A_log, dt_bias)
     if entry == "gdn_chunk_fwd" and q.dtype != torch.bfloat16:
         # The chunk kernels stage bf16 MFMA operands. fp32/fp16 q/k/v keep their precision on the
-        # recurrent kernel, which computes the same recurrence token by token in fp32.
+        # recurrent kernel, which computes the same recurrence in fp32.
         _note_recurrent_route(name, q.dtype)
         entry = "gdn_recurrent_fwd"
     grad_inputs = [q, k, v, g, beta, initial_state] + ([a_log_in, dt_bias_in] if use_gate_in_kernel else [])
