@@ -48,6 +48,7 @@ import itertools
 import json
 import os
 import platform
+import statistics
 import subprocess
 import sys
 import time
@@ -192,8 +193,7 @@ def block_pair(torch, steps: int) -> dict:
             for _ in range(2):
                 fn()
             settle(torch, fn)
-            ms, _ = time_launches(torch, fn, steps)
-            out[f"{name}_ms"] = round(ms, 4)
+            out[f"{name}_ms"] = round(median_time(torch, fn, steps), 4)
         # the attention kernel alone on the layer's own q, k, v, gate
         proj = torch.nn.functional.linear(x, attn._fused_weight(torch.bfloat16))
         nq, nkv = H * Dh, HKV * Dh
@@ -223,7 +223,7 @@ def block_pair(torch, steps: int) -> dict:
         for name, fn in ops_.items():
             fn()
             settle(torch, fn)
-            ms, _ = time_launches(torch, fn, steps)
+            ms = median_time(torch, fn, steps)
             out[f"{name}_ms"] = round(ms, 4)
     pair_ms = out["gdn_layer_ms"] + out["attn_layer_ms"]
     out.update({
@@ -255,6 +255,12 @@ def time_launches(torch, fn, steps: int, indexed: bool = False) -> tuple[float, 
     torch.cuda.synchronize()
     per_launch = sum(s.elapsed_time(e) for s, e in zip(starts, ends)) / steps
     return e0.elapsed_time(e1) / steps, per_launch
+
+
+def median_time(torch, fn, steps: int) -> float:
+    """Median over five runs of the mean ms per step: pauses of the host of tens of ms, which some processes meet once
+    or twice in their first runs, fall inside a mean of a few short calls."""
+    return statistics.median(time_launches(torch, fn, steps)[0] for _ in range(5))
 
 
 def time_back_to_back(torch, fn, steps: int, indexed: bool = False) -> float:
