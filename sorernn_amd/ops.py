@@ -598,9 +598,12 @@ def _chunk_qk(q: Tensor, k: Tensor, n: int, hv: int, vd: int, tokens: int, flags
     ``l2norm``'s, whose IEEE root and quotient can round to the next bf16. In other calls the choice of the route does
     not change the result: they are bit for bit the rows that the chunk kernels make, and calls that something watches,
     or whose rows are not 16-byte aligned, keep the norm in the kernels."""
+    long = 2 * n * hv * max(1, vd // 32) <= _cus(q) and tokens >= 2048 * n
+    if not long and torch.compiler.is_compiling():  # no guards on the length from the cost rule
+        return q, k, flags
     if not _l2norm_first(q, n, hv, vd, tokens):
         return q, k, flags
-    if 2 * n * hv * max(1, vd // 32) <= _cus(q) and tokens >= 2048 * n:
+    if long:
         q, k = _l2norm_qk(q, k)
         return q, k, flags & ~_lib.FLAG_QK_L2NORM
     if not _plain_eager(q, k):

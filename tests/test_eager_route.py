@@ -196,6 +196,10 @@ def test_watched_chunk_calls_keep_the_qk_norm_in_the_kernels(launches, monkeypat
     with SeenFunctions():
         q, k, flags = ops._chunk_qk(x, x, 1, 16, 128, 1000, 7)
     assert flags == 7 and q is x and k is x and len(calls) == 1
+    asked = []
+    monkeypatch.setattr(ops, "_l2norm_first", lambda *a: asked.append(a) or True)
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert ops._chunk_qk(x, x, 1, 16, 128, 1000, 7)[2] == 7 and not asked  # a compiled graph's guards: none on 1000
 
 
 @pytest.mark.parametrize("which", range(4))
