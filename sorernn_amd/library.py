@@ -20,39 +20,43 @@ from typing import Optional
 import torch
 from torch import Tensor
 from torch.autograd import forward_ad, profiler
-from torch._C import _functorch, _get_tracing_state, _is_torch_function_mode_enabled
+from torch._C import _dispatch_tls_is_dispatch_key_included as _tls_key_included
+from torch._C import _functorch, _is_torch_function_mode_enabled, _is_tracing, _len_torch_dispatch_stack
 from torch.fx import _symbolic_trace
 from torch.nn import Parameter
-from torch.utils import _python_dispatch
 
 from sorernn_amd import _lib
 
 C = 64  # chunk length
 
 
-def ordinary(*tensors) -> bool:
-    """True for ordinary tensors outside compile, FX tracing and dispatch modes: their values exist when a call returns."""
-    if torch.compiler.is_compiling():
-        return False
+_VMAP_MODE = torch._C._dispatch_key_parse("VmapMode")
+
+
+def _ordinary(tensors) -> bool:
     for t in tensors:
         if t is not None and type(t) is not Tensor and type(t) is not Parameter:
             return False
-    return not _symbolic_trace._is_fx_tracing_flag and _python_dispatch._get_current_dispatch_mode() is None
+    return not _symbolic_trace._is_fx_tracing_flag and _len_torch_dispatch_stack() == 0
+
+
+def ordinary(*tensors) -> bool:
+    """True for ordinary tensors outside compile, FX tracing and dispatch modes: their values exist when a call returns."""
+    return not torch.compiler.is_compiling() and _ordinary(tensors)
+
+
+def unwatched() -> bool:
+    """True when nothing but the autograd engine looks at the operators of ordinary tensors: no ``torch.jit`` tracing,
+    no functorch transform (vmap, grad, jvp), no forward-mode level, not inside the vmap that ``is_grads_batched`` runs
+    under (the type of its batched tensors is ``Tensor``), no torch-function mode, and no running profiler (it records
+    the registered ops)."""
+    return (not profiler._is_profiler_enabled and forward_ad._current_level < 0 and not _is_torch_function_mode_enabled()
+            and not _is_tracing() and _functorch.peek_interpreter_stack() is None and not _tls_key_included(_VMAP_MODE))
 
 
 def plain_eager(*tensors) -> bool:
-    """True when nothing but the autograd engine looks at these tensors' operators: ``ordinary``, and no ``torch.jit``
-    tracing, no functorch transform (vmap, grad, jvp), no forward-mode level, no batched tensor of the vmap that
-    ``is_grads_batched`` runs under (its type is ``Tensor`` as well), no torch-function mode, and no running profiler
-    (it records the registered ops)."""
-    if not ordinary(*tensors):
-        return False
-    for t in tensors:
-        if t is not None and _functorch.is_legacy_batchedtensor(t):
-            return False
-    return (_functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
-            and _get_tracing_state() is None and not _is_torch_function_mode_enabled()
-            and not profiler._is_profiler_enabled)
+    """``ordinary`` and ``unwatched``: a call of these tensors may run an op's implementation directly."""
+    return ordinary(*tensors) and unwatched()
 
 
 def _eager_function(impl, setup, backward):
@@ -84,7 +88,7 @@ def _eager(op, impl, function, *args):
     if torch.compiler.is_compiling():
         return op(*args)
     tensors = [a for a in args if isinstance(a, Tensor)]
-    if not plain_eager(*tensors):
+    if not (_ordinary(tensors) and unwatched()):
         return op(*args)
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return function(*args)

@@ -179,8 +179,10 @@ def _gdn_call(entry, name, q, k, v, g, beta, scale, initial_state, output_final_
         # implementation directly, under grad through an autograd function of it: the dispatcher round
         # trip costs more host time than the kernel launches.
         # the fp16 operand range guard (sorernn_amd/range_guard.py) reads its flag in eager calls, whatever watches them
-        word = _range.before_call(q.device) if _library.ordinary(q) else None
-        op = _library.chunk_fwd_call if needs_grad else _library.chunk_fwd_impl if _plain_eager(q) else _library.chunk_fwd
+        eager = _library.ordinary(q)
+        word = _range.before_call(q.device) if eager else None
+        direct = _library.chunk_fwd_impl if eager and _library.unwatched() else _library.chunk_fwd
+        op = _library.chunk_fwd_call if needs_grad else direct
         o, final, _, _ = op(q, k, v, g, beta, initial_state, a_log_in if use_gate_in_kernel else None,
                             dt_bias_in if use_gate_in_kernel else None, cu_seqlens, scale, flags, n,
                             bool(output_final_state), needs_grad)

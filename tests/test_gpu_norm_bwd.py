@@ -111,3 +111,13 @@ def test_rms_parameter_gradients_of_saturated_gates(dtype):
     ref = (dy.double() * F.silu(g.double())).sum(0)
     err = ((got.double().cpu() - ref) / ref).abs().max().item()
     assert err <= 5 * 2.0**-24, err * 2**24
+
+
+def test_batched_gradients():
+    """``is_grads_batched``: the device's backward thread runs under the caller's vmap, once per gradient."""
+    gen = torch.Generator().manual_seed(3)
+    x, dy = (torch.randn(33, 128, generator=gen).bfloat16().to(DEV).requires_grad_(True), torch.randn(3, 33, 128, generator=gen))
+    dy, y = dy.bfloat16().to(DEV), l2norm(x)
+    (got,) = torch.autograd.grad(y, x, dy, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        assert torch.equal(got[i], torch.autograd.grad(y, x, dy[i], retain_graph=True)[0])
