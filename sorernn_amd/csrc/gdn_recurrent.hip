@@ -266,7 +266,7 @@ __global__ __launch_bounds__(256) void gated_delta_recurrent_short_kernel(RecPar
 //   What bounds it: the 3 K / 4 fp32 MFMAs of a step (K = 128: 96 x 32 cycles a wave) and, for few sequences, the
 // chain of a step (K S, x through LDS, the triangular solve, the update). bf16, 16 heads of 128: 16 sequences of 64
 // tokens 37 us against 194 for the kernel before it (a token at a time, two barriers each); fp32, 2 sequences of
-// 512 tokens 122 against 1390; 4 heads of 64, 256 tokens 45 against 384.
+// 512 tokens 122 against 1390; 4 heads of 64, 256 tokens 46 against 384.
 template <typename E, int KD, int VD>
 __global__ __launch_bounds__(512, sizeof(E) == 4 ? 2 : 4) void gated_delta_recurrent_kernel(RecParams p) {
   constexpr int C = 16, A = KD / 16, KP = KD + 4, P = C + 4;  // 16-byte rows, spread over the banks
